@@ -91,8 +91,9 @@ __device__ __forceinline__ float bhalf(u32x2 w, int i) {
     return bf((uint16_t)((i < 2 ? w.x : w.y) >> (16 * (i & 1))));
 }
 
-// The autoregressive head after layer 2 (h2 in hf, B-fragment order). Head tiles: tile 0
-// (verb logits rows 0-7, value row 16) staged with W2, the two t1 tiles at pieces [0, 2048).
+// The autoregressive head after layer 2 (h2 of NB sample blocks in hf, B-fragment order; with
+// one block the second's lanes repeat it and M ends before their rows). Head tiles: tile 0
+// (verb logits rows 0-7, value row 16) at `head`, the two t1 tiles at pieces [0, 2048) of `stage`.
 // Lane half h draws for sample block h (sample m0 + 32h + lr): it gathers the block's eight
 // verb logits from its partner lane (l ^ 32), draws the verb with u0, and the partner learns
 // it back; each lane then forms z = tanh(bf16(ht + ev[verb])) for its 32 hidden units of both
@@ -100,23 +101,26 @@ __device__ __forceinline__ float bhalf(u32x2 w, int i) {
 // one K = 64 MFMA chain gives the drawn verb's 25 target logits, which the lane halves gather
 // as they did the verb logits and draw with u1. Rounding follows the bf16 torch forward:
 // every linear output is rounded once after its bias, ht + ev and tanh are rounded to bf16.
-__device__ __forceinline__ void ar_epilogue(const u32x4 *stage, const uint16_t *bl, const bf16x8 (&hf)[2][16],
-                                            int lane, int lr, int lh, int m0, int M, uint32_t key0, uint32_t key1,
+template <int NB>
+__device__ __forceinline__ void ar_epilogue(const u32x4 *head, const u32x4 *stage, const uint16_t *bl,
+                                            const bf16x8 (&hf)[NB][16], int lane, int lr, int lh, int m0, int M,
+                                            uint32_t key0, uint32_t key1,
                                             uint32_t tstep, float *__restrict__ value, int64_t *__restrict__ actions,
                                             float *__restrict__ logp, const ArOut &ar) {
     floatx16 z0[2] = {}, z1[2] = {}, z2[2] = {};
     {
-        const u32x4 *w0p = stage + 8 * 16 * 64 + lane, *w1p = stage + lane, *w2p = stage + 16 * 64 + lane;
+        const u32x4 *w0p = head + lane, *w1p = stage + lane, *w2p = stage + 16 * 64 + lane;
 #pragma unroll
         for (int s = 0; s < 16; s++) {
             const bf16x8 f0 = as_bf(w0p[s * 64]), f1 = as_bf(w1p[s * 64]), f2 = as_bf(w2p[s * 64]);
 #pragma unroll
-            for (int a = 0; a < 2; a++) {
+            for (int a = 0; a < NB; a++) {
                 z0[a] = mfma(f0, hf[a][s], z0[a]);
                 z1[a] = mfma(f1, hf[a][s], z1[a]);
                 z2[a] = mfma(f2, hf[a][s], z2[a]);
             }
         }
+        if (NB == 1) z0[1] = z0[0], z1[1] = z1[0], z2[1] = z2[0];   // lane half 1 repeats block 0; its rows are past M
     }
     const uint16_t *b3l = bl + 512, *btl = bl + 544;
     const uint32_t hm = 0u - (uint32_t)lh;
@@ -151,10 +155,10 @@ __device__ __forceinline__ void ar_epilogue(const u32x4 *stage, const uint16_t *
     const int va[2] = {lh ? vq : v, lh ? v : vq};   // the drawn verbs of blocks 0 and 1 of sample row lr
 
     // t2's B operand: z of this lane's hidden units for both blocks
-    bf16x8 hz[2][4];
+    bf16x8 hz[NB][4];
     const uint16_t *evl = (const uint16_t *)(stage + (PAE - PA1) / 8);
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int a = 0; a < NB; a++)
 #pragma unroll
         for (int T = 0; T < 2; T++)
 #pragma unroll
@@ -180,8 +184,9 @@ __device__ __forceinline__ void ar_epilogue(const u32x4 *stage, const uint16_t *
         for (int s = 0; s < 4; s++) {
             const bf16x8 f = as_bf(w3p[s * 64]);
 #pragma unroll
-            for (int a = 0; a < 2; a++) zt[a] = mfma(f, hz[a][s], zt[a]);
+            for (int a = 0; a < NB; a++) zt[a] = mfma(f, hz[a][s], zt[a]);
         }
+        if (NB == 1) zt[1] = zt[0];
     }
     // target row 8g + 4lh + i of block a sits in register 4g + i; lane half h gathers block h's
     float tl[NT];
@@ -220,6 +225,94 @@ __device__ __forceinline__ void ar_epilogue(const u32x4 *stage, const uint16_t *
     for (int a = 0; a < 2; a++) {
         const int ma = m0 + 32 * a + lr;
         if (ma < M && lh == 0) value[ma] = val[a];
+    }
+}
+
+// The 17-row head after layer 2 (h2 of NB sample blocks in hf, B-fragment order; NB == 1 as in
+// ar_epilogue) and, with SAMPLE, the draw of every row. w3: the head's 16 fragments in LDS.
+template <bool SAMPLE, int NB>
+__device__ __forceinline__ void head_epilogue(const u32x4 *head, const uint16_t *bl, const bf16x8 (&hf)[NB][16],
+                                              int lane, int lr, int lh, int m0, int M, uint32_t key0, uint32_t key1,
+                                              uint32_t tstep, float *__restrict__ logits, float *__restrict__ value,
+                                              int64_t *__restrict__ actions, float *__restrict__ logp) {
+    // ---- head: z[a] lane (lr, lh) register r = output 8(r/4) + 4lh + r%4 of sample 32a + lr
+    floatx16 z[2] = {};
+    {
+        const u32x4 *w3 = head + lane;
+        bf16x8 fw[16];   // all 16 head fragments read first: one LDS wait instead of sixteen
+#pragma unroll
+        for (int s = 0; s < 16; s++) fw[s] = as_bf(w3[s * 64]);
+#pragma unroll
+        for (int s = 0; s < 16; s++)
+#pragma unroll
+            for (int a = 0; a < NB; a++) z[a] = mfma(fw[s], hf[a][s], z[a]);
+        if (NB == 1) z[1] = z[0];
+    }
+    const uint16_t *b3l = bl + 512;
+    // the head output is bf16 (rounded once after the bias), widened to fp32; for sample block
+    // a this lane holds logits 4lh..4lh+3 (o[a][0..3]) and 8+4lh..8+4lh+3 (o[a][4..7]), lane
+    // half 0 the value
+    float o[2][8], v[2];
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+#pragma unroll
+        for (int g = 0; g < 2; g++)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+                const uint32_t w = cvt2(z[a][4 * g + i] + bf(b3l[8 * g + 4 * lh + i]),
+                                        z[a][4 * g + i + 1] + bf(b3l[8 * g + 4 * lh + i + 1]));
+                o[a][4 * g + i] = __uint_as_float(w << 16);
+                o[a][4 * g + i + 1] = __uint_as_float(w & 0xFFFF0000u);
+            }
+        v[a] = __uint_as_float(cvt2(z[a][8] + bf(b3l[16]), 0.f) << 16);
+    }
+    if (SAMPLE) {
+        // lane half h samples block a = h: it keeps its own half of that block's row and
+        // receives the other half from its partner lane (l ^ 32), which sends the half of
+        // the partner's own block that this lane lacks
+        // value blends by mask (a ternary between array elements is turned into a run-time
+        // index into a stack copy of the array)
+        const uint32_t hm = 0u - (uint32_t)lh;
+        auto pick = [&](float if0, float if1) {
+            return __uint_as_float((__float_as_uint(if1) & hm) | (__float_as_uint(if0) & ~hm));
+        };
+        float p[8], l16[16];
+#pragma unroll
+        for (int j = 0; j < 8; j++) p[j] = __shfl_xor(pick(o[1][j], o[0][j]), 32);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            l16[i] = pick(o[0][i], p[i]);
+            l16[4 + i] = pick(p[i], o[1][i]);
+            l16[8 + i] = pick(o[0][4 + i], p[4 + i]);
+            l16[12 + i] = pick(p[4 + i], o[1][4 + i]);
+        }
+        const int m = m0 + 32 * lh + lr;
+        if (m < M) {
+            auto lg = [&](int j) {   // a select chain: no register array indexed at run time
+                float r = l16[0];
+#pragma unroll
+                for (int q = 1; q < 16; q++) r = j == q ? l16[q] : r;
+                return r;
+            };
+            int act;
+            float lp;
+            d1s::sample_core(lg, NA, key0, key1, tstep, (uint32_t)m, act, lp);
+            actions[m] = act;
+            logp[m] = lp;
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        const int m = m0 + 32 * a + lr;
+        if (m < M) {
+            if (!SAMPLE || logits) {
+#pragma unroll
+                for (int g = 0; g < 2; g++)
+                    *(float4 *)(logits + (size_t)m * NA + 8 * g + 4 * lh) =
+                        make_float4(o[a][4 * g], o[a][4 * g + 1], o[a][4 * g + 2], o[a][4 * g + 3]);
+            }
+            if (lh == 0) value[m] = v[a];
+        }
     }
 }
 
@@ -493,88 +586,199 @@ __global__ __launch_bounds__(256) void k_policy(const uint8_t *__restrict__ obs,
     }
 
     if constexpr (AR) {
-        ar_epilogue(stage, bl, hf, lane, lr, lh, m0, M, key0, key1, (t_dev ? *t_dev : 0u) + t_add, value, actions,
-                    logp, ar);
+        ar_epilogue<2>(stage + 8 * 16 * 64, stage, bl, hf, lane, lr, lh, m0, M, key0, key1, (t_dev ? *t_dev : 0u) + t_add,
+                       value, actions, logp, ar);
         return;
     }
-    // ---- head: z[a] lane (lr, lh) register r = output 8(r/4) + 4lh + r%4 of sample 32a + lr
-    floatx16 z[2] = {};
-    {
-        const u32x4 *w3 = stage + 8 * 16 * 64 + lane;
-        bf16x8 fw[16];   // all 16 head fragments read first: one LDS wait instead of sixteen
+    head_epilogue<SAMPLE, 2>(stage + 8 * 16 * 64, bl, hf, lane, lr, lh, m0, M, key0, key1, tstep, logits, value, actions,
+                             logp);
+}
+
+// The same forward for small batches. k_policy gives a workgroup 256 samples, so a batch of
+// 1,024 ran on 4 of the 256 CUs and of 16,384 on 64, each for the whole 48 us that one wave per
+// SIMD needs for 256 samples. Here a workgroup owns 32 TB samples (TB = 1 or 2) and its eight
+// waves split the hidden units: wave w computes units 32w..32w+31 of every layer for all of
+// them. A wave then reads only its own row block's weight fragments, which go from L2 straight
+// to registers (a ring, three or five chunks ahead), while the observations, which every wave
+// needs, are widened once into fragment-ordered LDS. What bounds it is the stream of all of W1
+// (928 KB, 6 us at a CU's 64 B/clk) into each CU and the serial chain of loads, layers and the
+// draw, not MFMA work or the ring's depth. k_policy -> here, forward + sample: 46.5 -> 14.1 us
+// at 1,024 rows, 46.9 -> 18.1 at 8,192 (TB = 1), 47.1 -> 26.1 at 16,384 (TB = 2); with the
+// autoregressive head 57.4 -> 19.1, 58.1 -> 23.7 and 60.4 -> 33.8.
+//   x      the rows' bytes are all loaded at the start (16 bytes a lane and piece) and stored
+//          as widened fragments, 64 KB of chunks a phase into two buffers; TB = 1 fits both
+//          of its phases, TB = 2 stores phase p + 2 where phase p was.
+//   h1, h2 leave a wave as the two B fragments (K steps 2w, 2w + 1) that to_frags of k_policy
+//          builds, through LDS; the same packed weights, K order and accumulation order give
+//          bit-identical outputs.
+//   head   wave 0 alone (both sample blocks at TB = 2), with k_policy's epilogues.
+template <int MODE, int TB>
+__global__ __launch_bounds__(512) void k_policy_small(const uint8_t *__restrict__ obs, int M,
+                                                      const uint16_t *__restrict__ wpk, const uint16_t *__restrict__ b1,
+                                                      const uint16_t *__restrict__ b2, const uint16_t *__restrict__ b3,
+                                                      float *__restrict__ logits, float *__restrict__ value,
+                                                      uint32_t key0, uint32_t key1, const uint32_t *__restrict__ t_dev,
+                                                      uint32_t t_add, int64_t *__restrict__ actions,
+                                                      float *__restrict__ logp, ArOut ar) {
+    constexpr bool SAMPLE = MODE == 1, AR = MODE == 2;
+    constexpr int CP = 16 / TB, NP = (28 + CP - 1) / CP;   // 64-input chunks a phase, phases (chunks 0..27)
+    constexpr int PQ = CP * 4 * TB * 64;                   // 16-byte pieces of a phase buffer (64 KB)
+    constexpr int XT = TB * 64;                            // pieces of chunk 28's one used step
+    constexpr int HF = TB * 16 * 64;                       // pieces of one layer's output fragments
+    // after layer 1 the phase buffers hold h1 | h2 | head | AR pieces
+    constexpr int O_H2 = HF, O_HEAD = 2 * HF, O_AR = O_HEAD + 16 * 64;
+    static_assert(PQ == 4096 && O_AR + NSTAGE_AR <= 2 * PQ, "the later layers fit the phase buffers");
+    static_assert(TB == 2 || NP == 2, "TB = 1 keeps every phase in LDS");
+    __shared__ __align__(16) u32x4 xs[2 * PQ + XT];
+    __shared__ __align__(16) uint16_t bl[AR ? 640 : 544];   // b1 | b2 | head bias (32) | t1 bias (64) | t2 bias (32)
+    const int t = threadIdx.x, lane = t & 63, lr = lane & 31, lh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int m0 = blockIdx.x * 32 * TB;
+    const uint32_t tstep = MODE == 0 ? 0u : (t_dev ? *t_dev : 0u) + t_add;   // read early, as in k_policy
+
+    // layer-1 weights of chunk ch, row block `wave`: four consecutive 1 KB fragments
+    constexpr int RD = TB == 2 ? 6 : 4;   // ring slots (deeper ones gain nothing at TB = 1)
+    u32x4 wr[RD][4];
+    auto wload = [&](u32x4 (&w)[4], int ch) {
+        const u32x4 *src = (const u32x4 *)(wpk + PW1) + ((size_t)(ch * 8 + wave) * 4) * 64 + lane;
 #pragma unroll
-        for (int s = 0; s < 16; s++) fw[s] = as_bf(w3[s * 64]);
-#pragma unroll
-        for (int s = 0; s < 16; s++)
-#pragma unroll
-            for (int a = 0; a < 2; a++) z[a] = mfma(fw[s], hf[a][s], z[a]);
-    }
-    const uint16_t *b3l = bl + 512;
-    // the head output is bf16 (rounded once after the bias), widened to fp32; for sample block
-    // a this lane holds logits 4lh..4lh+3 (o[a][0..3]) and 8+4lh..8+4lh+3 (o[a][4..7]), lane
-    // half 0 the value
-    float o[2][8], v[2];
-#pragma unroll
-    for (int a = 0; a < 2; a++) {
-#pragma unroll
-        for (int g = 0; g < 2; g++)
-#pragma unroll
-            for (int i = 0; i < 4; i += 2) {
-                const uint32_t w = cvt2(z[a][4 * g + i] + bf(b3l[8 * g + 4 * lh + i]),
-                                        z[a][4 * g + i + 1] + bf(b3l[8 * g + 4 * lh + i + 1]));
-                o[a][4 * g + i] = __uint_as_float(w << 16);
-                o[a][4 * g + i + 1] = __uint_as_float(w & 0xFFFF0000u);
-            }
-        v[a] = __uint_as_float(cvt2(z[a][8] + bf(b3l[16]), 0.f) << 16);
-    }
-    if (SAMPLE) {
-        // lane half h samples block a = h: it keeps its own half of that block's row and
-        // receives the other half from its partner lane (l ^ 32), which sends the half of
-        // the partner's own block that this lane lacks
-        // value blends by mask (a ternary between array elements is turned into a run-time
-        // index into a stack copy of the array)
-        const uint32_t hm = 0u - (uint32_t)lh;
-        auto pick = [&](float if0, float if1) {
-            return __uint_as_float((__float_as_uint(if1) & hm) | (__float_as_uint(if0) & ~hm));
-        };
-        float p[8], l16[16];
-#pragma unroll
-        for (int j = 0; j < 8; j++) p[j] = __shfl_xor(pick(o[1][j], o[0][j]), 32);
+        for (int q = 0; q < 4; q++) w[q] = src[64 * q];
+    };
+    // piece i of phase p: row group rg of 16 rows, chunk cl of the phase; lane = row | 16-byte
+    // unit u of the row's 64 (half u >> 1, steps 2 (u & 1) and + 1). Rows at or past M read row
+    // M - 1, their outputs are not stored; rows start at multiples of 8 bytes.
+    typedef u32x4 __attribute__((aligned(8))) u32x4_a8;
+    const int r16 = lane & 15, u = lane >> 4;
+    u32x4 xv[NP][4];
+    auto xload = [&](u32x4 (&v)[4], int p) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            l16[i] = pick(o[0][i], p[i]);
-            l16[4 + i] = pick(p[i], o[1][i]);
-            l16[8 + i] = pick(o[0][4 + i], p[4 + i]);
-            l16[12 + i] = pick(p[4 + i], o[1][4 + i]);
+            const int g = wave + 8 * i, rg = g & (2 * TB - 1), ch = CP * p + g / (2 * TB);
+            const int row = min(m0 + 16 * rg + r16, M - 1);
+            if (ch < 28) v[i] = *(const u32x4_a8 *)(obs + (size_t)row * K1 + 64 * ch + 16 * u);
         }
-        const int m = m0 + 32 * lh + lr;
-        if (m < M) {
-            auto lg = [&](int j) {   // a select chain: no register array indexed at run time
-                float r = l16[0];
+    };
+    auto xstore = [&](const u32x4 (&v)[4], int p) {
+        u32x4 *dst = xs + (p & 1) * PQ;
 #pragma unroll
-                for (int q = 1; q < 16; q++) r = j == q ? l16[q] : r;
-                return r;
-            };
-            int act;
-            float lp;
-            d1s::sample_core(lg, NA, key0, key1, tstep, (uint32_t)m, act, lp);
-            actions[m] = act;
-            logp[m] = lp;
+        for (int i = 0; i < 4; i++) {
+            const int g = wave + 8 * i, rg = g & (2 * TB - 1), cl = g / (2 * TB);
+            if (CP * p + cl >= 28) continue;
+            const int slot = 16 * (rg & 1) + r16 + 32 * (u >> 1);
+            u32x4 *d = dst + ((cl * 4 + 2 * (u & 1)) * TB + (rg >> 1)) * 64 + slot;
+            d[0] = __builtin_bit_cast(u32x4, widen8(v[i].x, v[i].y));
+            d[TB * 64] = __builtin_bit_cast(u32x4, widen8(v[i].z, v[i].w));
+        }
+    };
+    xload(xv[0], 0);
+    u32x2 xt = {0u, 0u};
+    if (t < 32 * TB) xt = *(const u32x2 *)(obs + (size_t)min(m0 + t, M - 1) * K1 + 1792);
+#pragma unroll
+    for (int p = 1; p < NP; p++) xload(xv[p], p);
+#pragma unroll
+    for (int c = 0; c + 1 < RD; c++) wload(wr[c], c);
+    if (t < 256) bl[t] = b1[t];
+    else bl[t] = b2[t - 256];
+    if (t < 32) bl[512 + t] = t < NZ ? b3[t] : 0;
+    if (AR && t < TH + 32) bl[544 + t] = t < TH + NT ? ar.bt[t] : 0;
+    xstore(xv[0], 0);
+    xstore(xv[1], 1);
+    if (t < 32 * TB) {   // chunk 28, step 0: half 0 holds inputs 1792..1799, half 1 is zero
+        u32x4 *d = xs + 2 * PQ + (t >> 5) * 64 + (t & 31);
+        d[0] = __builtin_bit_cast(u32x4, widen8(xt.x, xt.y));
+        d[32] = u32x4{0u, 0u, 0u, 0u};
+    }
+    __syncthreads();
+
+    // ---- layer 1: chunk ch's weights sit in ring slot ch % RD
+    floatx16 acc[TB];
+#pragma unroll
+    for (int a = 0; a < TB; a++) acc[a] = floatx16{};
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+#pragma unroll
+        for (int cl = 0; cl < CP; cl++) {
+            const int ch = CP * p + cl;
+            if (ch >= 28) break;
+            if (ch + RD - 1 < C1) wload(wr[(ch + RD - 1) % RD], ch + RD - 1);
+            const u32x4 *src = xs + (p & 1) * PQ + cl * 4 * TB * 64 + lane;
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int a = 0; a < TB; a++) acc[a] = mfma(as_bf(wr[ch % RD][q]), as_bf(src[(q * TB + a) * 64]), acc[a]);
+        }
+        if (TB == 2 && p + 1 < NP) {
+            __syncthreads();   // phase p is read, phase p + 1 visible
+            if (p + 2 < NP) xstore(xv[p + 2], p + 2);
         }
     }
+    // this row block's layer-2 fragments, the head and the AR pieces, in flight from here
+    u32x4 w2f[16];
 #pragma unroll
-    for (int a = 0; a < 2; a++) {
-        const int m = m0 + 32 * a + lr;
-        if (m < M) {
-            if (!SAMPLE || logits) {
+    for (int s = 0; s < 16; s++) w2f[s] = ((const u32x4 *)(wpk + PW2))[(wave * 16 + s) * 64 + lane];
+    u32x4 hd[2];
 #pragma unroll
-                for (int g = 0; g < 2; g++)
-                    *(float4 *)(logits + (size_t)m * NA + 8 * g + 4 * lh) =
-                        make_float4(o[a][4 * g], o[a][4 * g + 1], o[a][4 * g + 2], o[a][4 * g + 3]);
+    for (int i = 0; i < 2; i++) hd[i] = ((const u32x4 *)(wpk + PW3))[t + 512 * i];
+    constexpr int RA = AR ? (NSTAGE_AR + 511) / 512 : 1;
+    u32x4 av[RA];
+    if (AR) {
+#pragma unroll
+        for (int i = 0; i < RA; i++) av[i] = ((const u32x4 *)(wpk + PA1))[min(t + 512 * i, NSTAGE_AR - 1)];
+    }
+#pragma unroll
+    for (int a = 0; a < TB; a++)   // chunk 28's other steps have zero weights
+        acc[a] = mfma(as_bf(wr[28 % RD][0]), as_bf(xs[2 * PQ + a * 64 + lane]), acc[a]);
+    __syncthreads();   // every wave is done with the x buffers
+
+    // bias + ReLU + bf16 rounding of acc into K steps 2 wave, 2 wave + 1 of the next layer
+    auto to_lds = [&](const uint16_t *bias, u32x4 *dst) {
+#pragma unroll
+        for (int a = 0; a < TB; a++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                u32x4 w;
+#pragma unroll
+                for (int k = 0; k < 2; k++) {   // registers 4g..4g+3: units 32 wave + 8g + 4lh + 0..3
+                    const int g = 2 * e + k;
+                    const u32x2 b = *(const u32x2 *)(bias + 32 * wave + 8 * g + 4 * lh);
+                    w[2 * k] = cvt2(fmaxf(acc[a][4 * g] + bhalf(b, 0), 0.f), fmaxf(acc[a][4 * g + 1] + bhalf(b, 1), 0.f));
+                    w[2 * k + 1] = cvt2(fmaxf(acc[a][4 * g + 2] + bhalf(b, 2), 0.f), fmaxf(acc[a][4 * g + 3] + bhalf(b, 3), 0.f));
+                }
+                dst[(a * 16 + 2 * wave + e) * 64 + lane] = w;
             }
-            if (lh == 0) value[m] = v[a];
-        }
+    };
+    to_lds(bl, xs);
+#pragma unroll
+    for (int i = 0; i < 2; i++) xs[O_HEAD + t + 512 * i] = hd[i];
+    if (AR) {
+#pragma unroll
+        for (int i = 0; i < RA; i++)
+            if (t + 512 * i < NSTAGE_AR) xs[O_AR + t + 512 * i] = av[i];
     }
+    __syncthreads();
+
+    // ---- layer 2
+#pragma unroll
+    for (int a = 0; a < TB; a++) acc[a] = floatx16{};
+#pragma unroll
+    for (int s = 0; s < 16; s++)
+#pragma unroll
+        for (int a = 0; a < TB; a++) acc[a] = mfma(as_bf(w2f[s]), as_bf(xs[(a * 16 + s) * 64 + lane]), acc[a]);
+    to_lds(bl + 256, xs + O_H2);
+    __syncthreads();
+    if (wave) return;
+
+    bf16x8 hf[TB][16];
+#pragma unroll
+    for (int a = 0; a < TB; a++)
+#pragma unroll
+        for (int s = 0; s < 16; s++) hf[a][s] = as_bf(xs[O_H2 + (a * 16 + s) * 64 + lane]);
+    const int me = min(M, m0 + 32 * TB);
+    if constexpr (AR)
+        ar_epilogue<TB>(xs + O_HEAD, xs + O_AR, bl, hf, lane, lr, lh, m0, me, key0, key1, tstep, value, actions, logp, ar);
+    else
+        head_epilogue<SAMPLE, TB>(xs + O_HEAD, bl, hf, lane, lr, lh, m0, me, key0, key1, tstep, logits, value, actions,
+                                  logp);
 }
 
 // Packed weights, one thread per element (gather form: every element is written, padding
@@ -622,6 +826,27 @@ __global__ __launch_bounds__(256) void k_policy_pack_ar(const uint16_t *__restri
     }
 }
 
+// Which kernel runs a batch of M rows. The lines are where a kernel's workgroups stop fitting
+// the 256 CUs at once (LDS allows each one a CU): 256 x 32 rows, then 256 x 64; past them the
+// next kernel wins at once (8,224 rows: 29.6 us with TB = 1, 21.4 with TB = 2; 16,416: 45.8
+// with TB = 2, 47.1 on k_policy, which from there on also keeps the fewest CU-microseconds a
+// row: callers run two such batches side by side).
+constexpr int SMALL1 = 8192, SMALL2 = 16384;
+template <int MODE>
+static int launch_policy(const uint8_t *obs, int M, const void *wpk, const void *b1, const void *b2, const void *b3,
+                         float *logits, float *value, uint64_t seed, const uint32_t *t_dev, uint32_t t_add,
+                         int64_t *actions, float *logp, const ArOut &ar, void *stream) {
+    auto go = [&](auto *kernel, int rows, int lanes) {
+        hipLaunchKernelGGL(kernel, dim3((M + rows - 1) / rows), dim3(lanes), 0, (hipStream_t)stream, obs, M,
+                           (const uint16_t *)wpk, (const uint16_t *)b1, (const uint16_t *)b2, (const uint16_t *)b3, logits,
+                           value, (uint32_t)seed, (uint32_t)(seed >> 32), t_dev, t_add, actions, logp, ar);
+    };
+    if (M <= SMALL1) go(k_policy_small<MODE, 1>, 32, 512);
+    else if (M <= SMALL2) go(k_policy_small<MODE, 2>, 64, 512);
+    else go(k_policy<MODE>, BM, 256);
+    return (int)hipGetLastError();
+}
+
 }  // namespace d1t
 
 extern "C" int64_t d1_policy_packed_elems(void) { return d1t::PEND; }
@@ -647,10 +872,7 @@ extern "C" int d1_policy_fwd_sample_ar(const uint8_t *obs, int M, const void *wp
         return D1_E_ARG;
     if (M == 0) return 0;
     const d1t::ArOut ar{(const uint16_t *)bt, verb, target, verb_logits, target_logits};
-    hipLaunchKernelGGL(d1t::k_policy<2>, dim3((M + d1t::BM - 1) / d1t::BM), dim3(256), 0, (hipStream_t)stream, obs, M,
-                       (const uint16_t *)wpk, (const uint16_t *)b1, (const uint16_t *)b2, (const uint16_t *)b3, nullptr,
-                       value, (uint32_t)seed, (uint32_t)(seed >> 32), t_dev, t_add, action, logp, ar);
-    return (int)hipGetLastError();
+    return d1t::launch_policy<2>(obs, M, wpk, b1, b2, b3, nullptr, value, seed, t_dev, t_add, action, logp, ar, stream);
 }
 
 extern "C" int d1_policy_pack(const void *w1, const void *w2, const void *w3, void *wpk, void *stream) {
@@ -665,10 +887,8 @@ extern "C" int d1_policy_fwd(const uint8_t *obs, int M, const void *wpk, const v
     if (M < 0 || (M > 0 && (!obs || !wpk || !b1 || !b2 || !b3 || !logits || !value))) return D1_E_ARG;
     if ((uintptr_t)obs % 8 || (uintptr_t)wpk % 16 || (uintptr_t)logits % 16) return D1_E_ARG;
     if (M == 0) return 0;
-    hipLaunchKernelGGL(d1t::k_policy<0>, dim3((M + d1t::BM - 1) / d1t::BM), dim3(256), 0, (hipStream_t)stream, obs,
-                       M, (const uint16_t *)wpk, (const uint16_t *)b1, (const uint16_t *)b2, (const uint16_t *)b3, logits,
-                       value, 0u, 0u, nullptr, 0u, nullptr, nullptr, d1t::ArOut{});
-    return (int)hipGetLastError();
+    return d1t::launch_policy<0>(obs, M, wpk, b1, b2, b3, logits, value, 0, nullptr, 0, nullptr, nullptr, d1t::ArOut{},
+                                 stream);
 }
 
 extern "C" int d1_policy_fwd_sample(const uint8_t *obs, int M, const void *wpk, const void *b1, const void *b2,
@@ -677,8 +897,6 @@ extern "C" int d1_policy_fwd_sample(const uint8_t *obs, int M, const void *wpk, 
     if (M < 0 || (M > 0 && (!obs || !wpk || !b1 || !b2 || !b3 || !value || !actions || !logp))) return D1_E_ARG;
     if ((uintptr_t)obs % 8 || (uintptr_t)wpk % 16 || (uintptr_t)logits % 16) return D1_E_ARG;
     if (M == 0) return 0;
-    hipLaunchKernelGGL(d1t::k_policy<1>, dim3((M + d1t::BM - 1) / d1t::BM), dim3(256), 0, (hipStream_t)stream, obs,
-                       M, (const uint16_t *)wpk, (const uint16_t *)b1, (const uint16_t *)b2, (const uint16_t *)b3, logits,
-                       value, (uint32_t)seed, (uint32_t)(seed >> 32), t_dev, t_add, actions, logp, d1t::ArOut{});
-    return (int)hipGetLastError();
+    return d1t::launch_policy<1>(obs, M, wpk, b1, b2, b3, logits, value, seed, t_dev, t_add, actions, logp,
+                                 d1t::ArOut{}, stream);
 }
