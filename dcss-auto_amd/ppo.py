@@ -193,7 +193,8 @@ class FastPPO:
         so the next step takes perm[0:minibatch]."""
         if self.perm is None or self.perm.shape != perm.shape:
             self.perm = torch.empty_like(perm, dtype=torch.int64)
-        self.perm.copy_(perm)
+        if perm is not self.perm:
+            self.perm.copy_(perm)
         self.cursor.zero_()
 
     def _step(self, obs, actions, logp, adv, ret):
@@ -241,32 +242,37 @@ class FastPPO:
                 self._step(obs, actions, logp, self._adv, self._ret)
         self._g, self._g_buf, self._g_args = g, buf, args
 
-    def advantages(self, buf):
-        adv, ret = P.gae(buf.rewards, buf.dones, buf.values, buf.bootstrap, self.gamma, self.lam)
-        flat = adv.flatten()
-        return (flat - flat.mean()) / (flat.std() + 1e-8), ret.flatten()
+    def advantages(self, buf, adv=None, ret=None):
+        """The buffer's normalised advantages and its returns, flat (written to `adv` and `ret`
+        when given)."""
+        n = buf.T * buf.N
+        if adv is None:
+            adv, ret = (torch.empty(n, dtype=torch.float32, device=self.dev) for _ in range(2))
+        return P.gae_normalized(buf.rewards, buf.dones, buf.values, buf.bootstrap, self.gamma, self.lam, adv, ret)
 
     def update(self, buf, generator=None):
-        adv, ret = self.advantages(buf)
         n = buf.T * buf.N
         obs, actions, logp = self._views(buf)
         if self.graph:
             if self._g is None or self._g_buf is not buf:
                 self._capture(buf)
-            self._adv.copy_(adv)
-            self._ret.copy_(ret)
-            adv, ret = self._adv, self._ret
+            adv, ret = self.advantages(buf, self._adv, self._ret)
             if not self._packed:   # weights replaced outside the step (a checkpoint load): the graph
                 self._struct(obs, actions, logp, adv, ret)   # only replays, so rebuild its weight copies here
+        else:
+            adv, ret = self.advantages(buf)
         steps = n // self.minibatch            # a ragged tail is dropped (T*N is a multiple in C4)
         for _ in range(self.epochs):
-            self.set_order(torch.randperm(n, device=self.dev, generator=generator))
+            if self.perm is None or self.perm.numel() != n:
+                self.perm = torch.empty(n, dtype=torch.int64, device=self.dev)
+            self.set_order(torch.randperm(n, out=self.perm, generator=generator))
             if self.graph:
                 for _ in range(steps // self._graph_len(n)):
                     self._g.replay()
             else:
                 for _ in range(steps):
                     self._step(obs, actions, logp, adv, ret)
+        terms = self.loss_terms()   # queued before the wait for the step counter
         if self.nonfinite_steps():
             raise RuntimeError('Non-finite PPO loss')
-        return self.loss_terms()
+        return terms
