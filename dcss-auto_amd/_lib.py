@@ -62,9 +62,7 @@ def load():
         L.d1_wait_init.argtypes = [p, i, i, p, p, C.c_uint64, i, p]
         L.d1_wait_run.argtypes = [p, i, i, p, p, i, p, p]
         L.d1_gae.argtypes = [p, p, p, p, i, i, C.c_float, C.c_float, p, p, p]
-        L.d1_gae_norm_work_bytes.argtypes = [i]
-        L.d1_gae_norm_work_bytes.restype = C.c_int64
-        L.d1_gae_norm.argtypes = [p, p, p, p, i, i, C.c_float, C.c_float, C.c_float, p, p, p, C.c_int64, p]
+        L.d1_adv_norm.argtypes = [p, C.c_int64, p, p, C.c_float, p]
         L.d1_los_table.argtypes = [p, i, p, p, p]
         L.d1_distance_rows.argtypes = [p, p, i, p, p]
         L.d1_policy_packed_elems.argtypes = []

@@ -9,13 +9,9 @@
 extern "C" {
 #endif
 
-/* d1_gae followed by adv = (adv - mean) / (std + eps) over the whole [T, n] buffer with the
- * unbiased standard deviation (gpu-d1/scripts/run_ring_ablations.py:354-362): two launches,
- * moments in fp64. `work` holds d1_gae_norm_work_bytes(n) bytes, 8-byte aligned. */
-int64_t d1_gae_norm_work_bytes(int n);
-int d1_gae_norm(const float *reward, const uint8_t *done, const float *value, const float *bootstrap, int T, int n,
-                float gamma, float gamma_lambda, float eps, float *adv, float *returns, void *work, int64_t work_bytes,
-                void *stream);
+/* adv[0..count) = (adv - *mean) / (*std + eps) in fp32, in place (the whole-buffer advantage
+ * normalisation of gpu-d1/scripts/run_ring_ablations.py:362; mean and std are device scalars). */
+int d1_adv_norm(float *adv, int64_t count, const float *mean, const float *std, float eps, void *stream);
 
 #ifdef __cplusplus
 }

@@ -1,8 +1,8 @@
 // d1hip: rollout-side kernels that sit around the policy network on MI355X.
 //   k_sample — categorical sampling with the Philox counter RNG (one lane per env).
 //   k_gae    — reverse-time GAE scan (one lane per env, a workgroup's waves over T; each
-//              time step's loads and stores are coalesced across envs), HBM-bound; with the
-//              moments of the advantages for k_adv_norm, which normalises them.
+//              time step's loads and stores are coalesced across envs), HBM-bound.
+//   k_adv_norm — the update's advantage normalisation.
 // Built with -ffp-contract=off: GAE products are rounded separately, as the
 // reference's elementwise PyTorch ops are (gpu-d1/scripts/run_ring_ablations.py:354-360).
 #include <hip/hip_runtime.h>
@@ -46,30 +46,6 @@ __global__ __launch_bounds__(256) void k_sample_dev(const float *__restrict__ lo
     sample_row(logits, i, k, ld, key0, key1, *t_dev + t_add, actions, logp);
 }
 
-// Mean and sum of squared deviations of `n` values, merged pairwise (Chan, Golub, LeVeque:
-// "Updating formulae and a pairwise algorithm for computing sample variances") in fp64.
-struct Moments {
-    double n, mean, m2;
-};
-__device__ __forceinline__ Moments merge(const Moments &a, const Moments &b) {
-    const double n = a.n + b.n;
-    if (!(n > 0.0)) return a;
-    const double d = b.mean - a.mean;
-    return {n, a.mean + d * (b.n / n), a.m2 + b.m2 + d * d * (a.n * b.n / n)};
-}
-__device__ __forceinline__ double shfl_xor_f64(double v, int o) {
-    const int lo = __shfl_xor((int)(uint32_t)__double_as_longlong(v), o);
-    const int hi = __shfl_xor((int)(__double_as_longlong(v) >> 32), o);
-    return __longlong_as_double(((long long)hi << 32) | (uint32_t)lo);
-}
-// over the wave; every lane ends with a merge in the same order of lanes up to mirrored pairs,
-// lane 0 with the one in lane order
-__device__ __forceinline__ Moments wave_merge(Moments x) {
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) x = merge(x, Moments{shfl_xor_f64(x.n, o), shfl_xor_f64(x.mean, o), shfl_xor_f64(x.m2, o)});
-    return x;
-}
-
 // Reverse-time GAE. A workgroup owns 64 envs (a lane each); its eight waves take GC time steps
 // each, so that a round's GW * GC = 128 steps are all in flight at once. Each wave forms its
 // steps' deltas, then the waves run the recurrence in time order, the carry passing through
@@ -77,19 +53,16 @@ __device__ __forceinline__ Moments wave_merge(Moments x) {
 // the reference's loop (bit-identical to it). One lane looping over T with a load level a step
 // left the kernel waiting on latency, 1,024 waves on the chip: 106.8 us at T = 128, n = 65,536
 // (143 MB) with the buffers out of cache, now 34.6 us (4.1 TB/s; a large copy reaches 5.1).
-// With STATS each workgroup also leaves the moments of its advantages in part[blockIdx.x].
 constexpr int GW = 8, GC = 16;
-template <bool STATS>
 __global__ __launch_bounds__(64 * GW) void k_gae(const float *reward, const uint8_t *done, const float *value,
                                                  const float *bootstrap, int T, int n, float gamma, float gl, float *adv,
-                                                 float *ret, Moments *part) {
+                                                 float *ret) {
     __shared__ float first[GW][64], carry[64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int env = blockIdx.x * 64 + lane;
     const bool mine = env < n;
     const int i = mine ? env : n - 1;
     float after = bootstrap[i];   // value of the step after the round's last one
-    Moments st{0.0, 0.0, 0.0};
     if (wave == 0) carry[lane] = 0.f;
     for (int base = T - 1; base >= 0; base -= GW * GC) {
         const int t0 = base - GC * wave;   // this wave's steps t0, t0 - 1, .. ; wave 0 has the latest
@@ -148,48 +121,15 @@ __global__ __launch_bounds__(64 * GW) void k_gae(const float *reward, const uint
                     adv[o] = r[j];
                     if (ret) ret[o] = r[j] + v[j];
                 }
-            if (STATS && cnt > 0) {   // two passes over the registers: exact up to fp64 rounding
-                double sum = 0.0, m2 = 0.0;
-#pragma unroll
-                for (int j = 0; j < GC; j++) sum += j < cnt ? (double)r[j] : 0.0;
-                const double mean = sum / (double)cnt;
-#pragma unroll
-                for (int j = 0; j < GC; j++) {
-                    const double e = (double)r[j] - mean;
-                    m2 += j < cnt ? e * e : 0.0;
-                }
-                st = merge(st, Moments{(double)cnt, mean, m2});
-            }
-        }
-    }
-    if (STATS) {
-        __shared__ Moments ws[GW];
-        st = wave_merge(st);
-        if (lane == 0) ws[wave] = st;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            Moments x = ws[0];
-            for (int w = 1; w < GW; w++) x = merge(x, ws[w]);
-            part[blockIdx.x] = x;
         }
     }
 }
 
-// adv = (adv - mean) / (std + eps) over the whole buffer (unbiased std, as torch.std), from the
-// workgroups' moments: every workgroup merges all of them in the same order (24 bytes each,
-// from L2), then normalises its slice. Mean and std are rounded to fp32 once. The update's
-// start was eight launches (GAE, mean, std, four elementwise passes, copies into the captured
-// buffers) and is two: 62 us less a small update (4 minibatches of 1,024: 331 -> 270 us).
-__global__ __launch_bounds__(256) void k_adv_norm(float *__restrict__ adv, int64_t count, const Moments *__restrict__ part,
-                                                  int parts, float eps) {
-    __shared__ Moments ws[4];
-    Moments x{0.0, 0.0, 0.0};
-    for (int q = threadIdx.x; q < parts; q += 256) x = merge(x, part[q]);
-    x = wave_merge(x);
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = x;
-    __syncthreads();
-    x = merge(merge(ws[0], ws[1]), merge(ws[2], ws[3]));
-    const float mean = (float)x.mean, den = (float)sqrt(x.m2 / (x.n - 1.0)) + eps;
+// adv = (adv - mean[0]) / (std[0] + eps) in place, each operation rounded to fp32 as the
+// elementwise chain rounds it (one pass over the buffer where the chain makes three).
+__global__ __launch_bounds__(256) void k_adv_norm(float *__restrict__ adv, int64_t count, const float *__restrict__ mean_p,
+                                                  const float *__restrict__ std_p, float eps) {
+    const float mean = *mean_p, den = *std_p + eps;
     const int64_t step = (int64_t)gridDim.x * 256, at = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if ((uintptr_t)adv % 16 == 0) {
         for (int64_t q = at; q < count / 4; q += step) {
@@ -323,24 +263,16 @@ int d1_gae(const float *reward, const uint8_t *done, const float *value, const f
            float gamma, float gamma_lambda, float *adv, float *returns, void *stream) {
     if (T < 0 || n < 0 || ((T && n) && (!reward || !done || !value || !bootstrap || !adv))) return D1_E_ARG;
     if (T == 0 || n == 0) return 0;
-    hipLaunchKernelGGL(d1p::k_gae<false>, dim3((n + 63) / 64), dim3(64 * d1p::GW), 0, (hipStream_t)stream, reward, done,
-                       value, bootstrap, T, n, gamma, gamma_lambda, adv, returns, nullptr);
+    hipLaunchKernelGGL(d1p::k_gae, dim3((n + 63) / 64), dim3(64 * d1p::GW), 0, (hipStream_t)stream, reward, done, value,
+                       bootstrap, T, n, gamma, gamma_lambda, adv, returns);
     return (int)hipGetLastError();
 }
-int64_t d1_gae_norm_work_bytes(int n) { return n < 0 ? D1_E_ARG : (int64_t)((n + 63) / 64) * (int64_t)sizeof(d1p::Moments); }
-int d1_gae_norm(const float *reward, const uint8_t *done, const float *value, const float *bootstrap, int T, int n,
-                float gamma, float gamma_lambda, float eps, float *adv, float *returns, void *work, int64_t work_bytes,
-                void *stream) {
-    if (T < 0 || n < 0 || ((T && n) && (!reward || !done || !value || !bootstrap || !adv || !work))) return D1_E_ARG;
-    if (T == 0 || n == 0) return 0;
-    if ((uintptr_t)work % 8 || work_bytes < d1_gae_norm_work_bytes(n)) return D1_E_ARG;
-    const int parts = (n + 63) / 64;
-    const int64_t count = (int64_t)T * n;
+int d1_adv_norm(float *adv, int64_t count, const float *mean, const float *std, float eps, void *stream) {
+    if (count < 0 || (count && (!adv || !mean || !std))) return D1_E_ARG;
+    if (count == 0) return 0;
     const int64_t groups = (count / 4 + 255) / 256;   // one float4 a lane, at most eight workgroups a CU
-    hipLaunchKernelGGL(d1p::k_gae<true>, dim3(parts), dim3(64 * d1p::GW), 0, (hipStream_t)stream, reward, done, value,
-                       bootstrap, T, n, gamma, gamma_lambda, adv, returns, (d1p::Moments *)work);
     hipLaunchKernelGGL(d1p::k_adv_norm, dim3((unsigned)(groups < 1 ? 1 : groups > 2048 ? 2048 : groups)), dim3(256), 0,
-                       (hipStream_t)stream, adv, count, (const d1p::Moments *)work, parts, eps);
+                       (hipStream_t)stream, adv, count, mean, std, eps);
     return (int)hipGetLastError();
 }
 }

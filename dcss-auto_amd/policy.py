@@ -162,18 +162,13 @@ def sample_dev(logits, seed, t_dev, t_add, actions, logp):
     return actions, logp
 
 
-def _check_gae(reward, done, value, bootstrap):
+def gae(reward, done, value, bootstrap, gamma=0.99, lam=0.95, adv=None, returns=None):
+    """HIP reverse-time GAE over [T, N] fp32 rewards/values and uint8 dones."""
     T, n = reward.shape
     for t_ in (reward, value):
         assert t_.dtype == torch.float32 and t_.is_contiguous() and t_.shape == (T, n)
     assert done.dtype == torch.uint8 and done.is_contiguous() and done.shape == (T, n)
     assert bootstrap.dtype == torch.float32 and bootstrap.shape == (n,) and bootstrap.is_contiguous()
-    return T, n
-
-
-def gae(reward, done, value, bootstrap, gamma=0.99, lam=0.95, adv=None, returns=None):
-    """HIP reverse-time GAE over [T, N] fp32 rewards/values and uint8 dones."""
-    T, n = _check_gae(reward, done, value, bootstrap)
     if adv is None:
         adv = torch.empty_like(reward)
     if returns is None:
@@ -185,20 +180,14 @@ def gae(reward, done, value, bootstrap, gamma=0.99, lam=0.95, adv=None, returns=
     return adv, returns
 
 
-def gae_normalized(reward, done, value, bootstrap, gamma, lam, adv, returns, eps=1e-8):
-    """gae() with the advantages normalised over the whole buffer, (adv - mean) / (std + eps)
-    with the unbiased std, in two launches: contiguous fp32 `adv` and `returns` of T * N
-    elements are written."""
-    T, n = _check_gae(reward, done, value, bootstrap)
-    for t_ in (adv, returns):
-        assert t_.dtype == torch.float32 and t_.is_contiguous() and t_.numel() == T * n and t_.device == reward.device
-    L = _lib.load()
-    nbytes = L.d1_gae_norm_work_bytes(n)
-    work = torch.empty(nbytes, dtype=torch.uint8, device=reward.device)
-    _lib.check(L.d1_gae_norm(reward.data_ptr(), done.data_ptr(), value.data_ptr(), bootstrap.data_ptr(), T, n,
-                             float(gamma), float(gamma * lam), float(eps), adv.data_ptr(), returns.data_ptr(),
-                             work.data_ptr(), nbytes, torch.cuda.current_stream(reward.device).cuda_stream), 'd1_gae_norm')
-    return adv, returns
+def normalize_(adv, eps=1e-8):
+    """adv = (adv - mean) / (std + eps) in place over the whole buffer (unbiased std), the bits of
+    the elementwise expression; contiguous fp32."""
+    assert adv.dtype == torch.float32 and adv.is_contiguous()
+    mean, std = adv.mean(), adv.std()
+    _lib.check(_lib.load().d1_adv_norm(adv.data_ptr(), adv.numel(), mean.data_ptr(), std.data_ptr(), float(eps),
+                                       torch.cuda.current_stream(adv.device).cuda_stream), 'd1_adv_norm')
+    return adv
 
 
 # ----------------------------------------------------------------------------------------

@@ -248,7 +248,8 @@ class FastPPO:
         n = buf.T * buf.N
         if adv is None:
             adv, ret = (torch.empty(n, dtype=torch.float32, device=self.dev) for _ in range(2))
-        return P.gae_normalized(buf.rewards, buf.dones, buf.values, buf.bootstrap, self.gamma, self.lam, adv, ret)
+        P.gae(buf.rewards, buf.dones, buf.values, buf.bootstrap, self.gamma, self.lam, adv=adv, returns=ret)
+        return P.normalize_(adv), ret
 
     def update(self, buf, generator=None):
         n = buf.T * buf.N
