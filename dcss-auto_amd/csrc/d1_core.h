@@ -33,7 +33,6 @@ struct Smem {
             // BFS layer mod 3 of every reached cell as two bit planes: lay0 = layer % 3 == 1,
             // lay1 = layer % 3 == 2. Cells that BFS-neighbour each other differ by at most one
             // layer, so their layers mod 3 fix the sign of every comparison the monster rules make
-            int32_t rowpre[72];   // inclusive per-row prefix counts (episode reset)
             uint32_t lay0[ROWS_WORDS];
             uint32_t lay1[ROWS_WORDS];
         };
@@ -60,7 +59,8 @@ __device__ __forceinline__ uint64_t ballot(bool b) { return __ballot(b); }
 template <int CTRL, int ROWS = 0xF>
 __device__ __forceinline__ int dpp(int v, int id) { return __builtin_amdgcn_update_dpp(id, v, CTRL, ROWS, 0xF, false); }
 constexpr int DPP_QUAD_1032 = 0xB1, DPP_QUAD_2301 = 0x4E, DPP_ROW_HALF_MIRROR = 0x141, DPP_ROW_MIRROR = 0x140,
-              DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143, DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138;
+              DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143, DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138,
+              DPP_ROW_SHR1 = 0x111, DPP_ROW_SHR2 = 0x112, DPP_ROW_SHR4 = 0x114, DPP_ROW_SHR8 = 0x118;
 // lane l <- l-1 / l+1; bound control makes lane 0 / lane 63 (no source lane) read 0
 __device__ __forceinline__ uint32_t lane_up(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, DPP_WAVE_SHR1, 0xF, 0xF, true);
@@ -90,6 +90,16 @@ __device__ __forceinline__ int wave_min(int v) {
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
     return (uint32_t)wave_reduce((int)v, 0, [](int a, int b) { return (int)((uint32_t)a + (uint32_t)b); });
 }
+// Inclusive prefix sum over the lanes (every lane active): within the rows of 16, then row 0's
+// total into row 1 and row 2's into row 3, then rows 0-1's into rows 2-3.
+__device__ __forceinline__ int wave_scan(int v) {
+    v += dpp<DPP_ROW_SHR1>(v, 0);
+    v += dpp<DPP_ROW_SHR2>(v, 0);
+    v += dpp<DPP_ROW_SHR4>(v, 0);
+    v += dpp<DPP_ROW_SHR8>(v, 0);
+    v += dpp<DPP_ROW_BCAST15, 0xA>(v, 0);
+    return v + dpp<DPP_ROW_BCAST31, 0xC>(v, 0);
+}
 // gpu-d1/src/sim.h:14
 __device__ __forceinline__ int cheb(int a, int b) { return imax(iabs(a % W - b % W), iabs(a / W - b / W)); }
 // the same for two cells of the map (0 <= a, b < N): unsigned division by the width is shorter
@@ -113,6 +123,9 @@ __device__ __forceinline__ bool bit(const uint32_t *bm, int p) { return bit_at(b
 struct Row {
     uint32_t a, b, c;   // bits 0-31, 32-63, 64-79
 };
+__device__ __forceinline__ Row row_lane(Row r, int l) {
+    return {(uint32_t)lane_val((int)r.a, l), (uint32_t)lane_val((int)r.b, l), (uint32_t)lane_val((int)r.c, l)};
+}
 __device__ __forceinline__ Row row_ld(const uint32_t *bm, int y) { return {bm[y * RW], bm[y * RW + 1], bm[y * RW + 2]}; }
 __device__ __forceinline__ void row_st(uint32_t *bm, int y, Row r) { bm[y * RW] = r.a; bm[y * RW + 1] = r.b; bm[y * RW + 2] = r.c; }
 __device__ __forceinline__ Row row_or(Row x, Row y) { return {x.a | y.a, x.b | y.b, x.c | y.c}; }
@@ -222,6 +235,21 @@ __device__ __noinline__ uint32_t philox_lane(uint32_t key0, uint32_t key1, uint3
     return j == 0 ? c0 : j == 1 ? c1 : j == 2 ? c2 : c3;
 }
 
+// all four words of block `blk` of the stream
+__device__ __forceinline__ void philox_block(uint32_t key0, uint32_t key1, uint32_t t, uint32_t env, uint32_t dom,
+                                             uint32_t blk, uint32_t (&w)[4]) {
+    uint32_t c0 = blk, c1 = t, c2 = env, c3 = dom, k0 = key0, k1 = key1;
+#pragma unroll
+    for (int r = 0; r < 10; r++) {
+        const uint32_t hi0 = __umulhi(0xD2511F53u, c0), lo0 = 0xD2511F53u * c0;
+        const uint32_t hi1 = __umulhi(0xCD9E8D57u, c2), lo1 = 0xCD9E8D57u * c2;
+        const uint32_t n0 = hi1 ^ c1 ^ k0, n2 = hi0 ^ c3 ^ k1;
+        c0 = n0; c1 = lo1; c2 = n2; c3 = lo0;
+        k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
+    }
+    w[0] = c0; w[1] = c1; w[2] = c2; w[3] = c3;
+}
+
 struct Rng {
     uint64_t st, inc;                   // PCG32: the state before draw `sb`
     uint32_t key0, key1, t, env, dom;   // counter stream
@@ -312,30 +340,54 @@ struct Rng {
 
 // Reservoir choice over `total` eligible cells: the 1-based count c is kept when
 // r(c) == 0, the last kept count wins (gpu-d1/branches/d1-stairs-v2/src/learn.cu:432-441).
-// 64 counts per pass: lane l evaluates count c0+l from the draw it would get if no
-// earlier draw in the pass were rejected (the buffer refilled at the current index);
-// a pass in which any Lemire rejection is possible (low < bound) is replayed serially,
-// so the draw sequence is the serial one.
+// Without a Lemire rejection count c takes draw c - 2 from here, so the counts are evaluated
+// side by side: in counter mode a lane's Philox block gives it four of them (256 a pass), in
+// PCG mode the lanes hold 64 consecutive states and all jump 64 ahead (no table load in the
+// loop). A draw that may be rejected (low < bound, about one choice in 20,000 at 700 cells)
+// has the whole choice replayed serially from the untouched generator. Filling the draw buffer
+// 64 counts at a time through its out-of-line generator, 700 cells took about 5 us of a reset.
 __device__ __forceinline__ int reservoir(Rng &s, int total, int lane) {
-    int chosen = total >= 1 ? 0 : -1;
-    int c0 = 2;
-    while (c0 <= total) {
-        int cnt = imin(64, total - c0 + 1);
-        int c = c0 + lane;
-        if (s.o != 0) s.fill(s.k());
-        uint64_t m = (uint64_t)s.buf * (uint32_t)c;
-        bool act = lane < cnt;
-        bool risky = act && (uint32_t)m < (uint32_t)c;
-        if (ballot(risky)) {
-            for (int cc = c0; cc < c0 + cnt; cc++) if (s.r(cc) == 0) chosen = cc - 1;
-        } else {
-            uint64_t keep = ballot(act && (m >> 32) == 0);
-            if (keep) chosen = c0 + 63 - __clzll((long long)keep) - 1;
-            s.o += (uint32_t)cnt;
+    if (total < 2) return total - 1;   // one cell: count 1 is kept without a draw; none: -1
+    const uint32_t nd = (uint32_t)total - 1u, k0 = s.k();   // draws k0 .. k0 + nd - 1
+    uint32_t best = 1;
+    bool risky = false;
+    auto test = [&](uint32_t w, uint32_t c) {   // a lane's counts ascend
+        const bool act = c - 2u < nd;
+        risky |= act && w * c < c;
+        best = act && __umulhi(w, c) == 0 ? c : best;
+    };
+    if (s.mode == 0) {
+        const uint32_t j = k0 - s.sb;
+        uint64_t st = kJump.a[j] * s.st + kJump.c[j] * s.inc;   // the state before draw k0
+        const uint64_t a64 = kJump.a[64], c64 = kJump.c[64] * s.inc;
+        uint64_t sl = kJump.a[lane] * st + kJump.c[lane] * s.inc;
+        for (uint32_t d = 0; d < nd; d += 64) {
+            test(pcg_out(sl), d + (uint32_t)lane + 2u);
+            sl = a64 * sl + c64;
         }
-        c0 += cnt;
+        if (!ballot(risky)) {
+            uint32_t d = 0;
+            for (; d + 64 <= nd; d += 64) st = a64 * st + c64;
+            s.st = st;
+            s.sb = k0 + d;
+        }
+    } else {
+        for (uint32_t blk = k0 >> 2; (int32_t)(4u * blk - k0) < (int32_t)nd; blk += 64) {
+            uint32_t w[4];
+            philox_block(s.key0, s.key1, s.t, s.env, s.dom, blk + (uint32_t)lane, w);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; q++) test(w[q], 4u * (blk + (uint32_t)lane) + q - k0 + 2u);
+        }
     }
-    return chosen;
+    if (ballot(risky)) {
+        int chosen = 0;
+        for (int c = 2; c <= total; c++)
+            if (s.r(c) == 0) chosen = c - 1;
+        return chosen;
+    }
+    s.base = k0 + nd - 64u;   // the next draw is k0 + nd, the buffer empty
+    s.o = 64;
+    return wave_max((int)best) - 1;
 }
 
 // ---------------------------------------------------------------- world context
@@ -531,28 +583,28 @@ __device__ __forceinline__ void occ_clear_lane(Ctx &x, int p) {
 }
 
 // ---------------------------------------------------------------- cell selection
-// Row prefix counts of a bitmap (rows in `bm`), stored inclusive in sm->rowpre.
-__device__ __forceinline__ int row_prefix(Ctx &x, const uint32_t *bm) {
-    int y0 = x.lane, y1 = x.lane + 64;
-    int c0 = row_popc(row_ld(bm, y0));
-    int c1 = y1 < H ? row_popc(row_ld(bm, y1)) : 0;
-    int s0 = c0;
-    for (int o = 1; o < 64; o <<= 1) { int v = __shfl_up(s0, o); if (x.lane >= o) s0 += v; }
-    int tot0 = lane_val(s0, 63);
-    int s1 = c1;
-    for (int o = 1; o < 64; o <<= 1) { int v = __shfl_up(s1, o); if (x.lane >= o) s1 += v; }
-    __syncthreads();
-    x.sm->rowpre[y0] = s0;
-    if (y1 < H) x.sm->rowpre[y1] = s1 + tot0;
-    __syncthreads();
-    return x.sm->rowpre[H - 1];
+// A bitmap in registers (lane l holds rows l and, l < 6, 64 + l; r1 is zero in the other lanes)
+// with the inclusive prefix counts of its rows.
+struct Rows {
+    Row r0, r1;
+    int p0, p1, tot0, total;
+};
+__device__ __forceinline__ Rows rows_count(Row r0, Row r1) {
+    Rows b{r0, r1, wave_scan(row_popc(r0)), wave_scan(row_popc(r1)), 0, 0};
+    b.tot0 = lane_val(b.p0, 63);
+    b.p1 += b.tot0;
+    b.total = lane_val(b.p1, 63);
+    return b;
 }
-// The k-th set cell (row-major) of bitmap `bm`, given its rowpre.
-__device__ __forceinline__ int select_cell(Ctx &x, const uint32_t *bm, int k) {
-    int lo = 0, hi = H - 1;   // first row with rowpre > k
-    while (lo < hi) { int mid = (lo + hi) >> 1; if (x.sm->rowpre[mid] > k) hi = mid; else lo = mid + 1; }
-    int before = lo ? x.sm->rowpre[lo - 1] : 0;
-    return lo * W + row_select(row_ld(bm, lo), k - before);
+// The k-th set cell (row-major), k < total uniform: a ballot finds its row and the rest runs on
+// that row's three words in scalar registers (a binary search over prefix counts in LDS waited
+// out seven LDS round trips a cell).
+__device__ __forceinline__ int rows_select(const Rows &b, int k) {
+    const uint64_t m0 = ballot(b.p0 > k), m = m0 ? m0 : ballot(b.p1 > k);
+    const int l = m ? __ffsll((unsigned long long)m) - 1 : 0;
+    const int before = m0 ? lane_val(b.p0, l) - row_popc(row_lane(b.r0, l)) : lane_val(b.p1, l) - row_popc(row_lane(b.r1, l));
+    const Row r = m0 ? row_lane(b.r0, l) : row_lane(b.r1, l);
+    return (m0 ? l : 64 + l) * W + row_select(r, k - before);
 }
 
 // ---------------------------------------------------------------- monsters
@@ -855,9 +907,6 @@ __device__ __forceinline__ int choose_move(Ctx &x, int id, int p, int plag, int 
 // phase reads them); the frontier bitmap is left clear for the repair search's marks.
 __device__ __forceinline__ Row row_up(Row r) { return {lane_up(r.a), lane_up(r.b), lane_up(r.c)}; }
 __device__ __forceinline__ Row row_dn(Row r) { return {lane_dn(r.a), lane_dn(r.b), lane_dn(r.c)}; }
-__device__ __forceinline__ Row row_lane(Row r, int l) {
-    return {(uint32_t)lane_val((int)r.a, l), (uint32_t)lane_val((int)r.b, l), (uint32_t)lane_val((int)r.c, l)};
-}
 __device__ __forceinline__ Row row_sel(bool c, Row x, Row y) { return c ? x : y; }
 __device__ __forceinline__ Row dilate(Row f, Row up, Row dn) {
     Row v = row_or(f, row_or(up, dn));
@@ -891,34 +940,46 @@ __device__ __forceinline__ void bfs(Ctx &x, uint64_t movers, int margin) {
     const uint32_t mbit = mover ? 1u << ((x.mpos % W) & 31) : 0u;
     x.mlay = FAR;
     int m3 = 0, stop = 1 << 30, last = 0;
+    // lanes with frontier cells in their first and second row: the second set is worked on only
+    // while the frontier is in or next to rows 64.. (lane 0 and lane 63 read zero rows past the
+    // wave's ends, and lane 6's second row is empty, so the map's edges need no masks)
+    uint64_t on0 = ballot(row_any(f0)), on1 = ballot(row_any(f1));
     for (int layer = 1; layer < N; layer++) {
         m3 = m3 == 2 ? 0 : m3 + 1;
-        const Row f0_63 = row_lane(f0, 63);
         Row n0, n1 = zero;
-        if (row_any(f0_63) || ballot(row_any(f1))) {   // rows 64.. can grow this layer
-            const Row f1_0 = row_lane(f1, 0);
-            const Row u0 = row_sel(lane == 0, zero, row_up(f0)), d0 = row_sel(lane == 63, f1_0, row_dn(f0));
-            const Row u1 = row_sel(lane == 0, f0_63, row_up(f1)), d1 = row_sel(lane >= H - 65, zero, row_dn(f1));
+        if ((on0 >> 63) | on1) {
+            const Row f1_0 = row_lane(f1, 0), f0_63 = row_lane(f0, 63);
+            const Row u0 = row_up(f0), d0 = row_sel(lane == 63, f1_0, row_dn(f0));
+            const Row u1 = row_sel(lane == 0, f0_63, row_up(f1)), d1 = row_dn(f1);
             n0 = row_andn(row_and(dilate(f0, u0, d0), fl0), r0);
-            n1 = has1 ? row_andn(row_and(dilate(f1, u1, d1), fl1), r1) : zero;
-        } else {   // no frontier in rows 63..: the second row set neither grows nor feeds row 63
-            const Row u0 = row_sel(lane == 0, zero, row_up(f0)), d0 = row_sel(lane == 63, zero, row_dn(f0));
-            n0 = row_andn(row_and(dilate(f0, u0, d0), fl0), r0);
+            n1 = row_andn(row_and(dilate(f1, u1, d1), fl1), r1);   // fl1 is zero in lanes 6..
+            r1 = row_or(r1, n1);
+            f1 = n1;
+            if (m3 == 1) a1 = row_or(a1, n1);
+            if (m3 == 2) b1 = row_or(b1, n1);
+            on1 = ballot(row_any(n1));
+        } else {
+            n0 = row_andn(row_and(dilate(f0, row_up(f0), row_dn(f0)), fl0), r0);
         }
-        if (!ballot(row_any(n0) || row_any(n1))) break;
+        on0 = ballot(row_any(n0));
+        if (!(on0 | on1)) break;
         last = layer;
-        r0 = row_or(r0, n0); r1 = row_or(r1, n1);
-        f0 = n0; f1 = n1;
-        if (m3 == 1) { a0 = row_or(a0, n0); a1 = row_or(a1, n1); }
-        if (m3 == 2) { b0 = row_or(b0, n0); b1 = row_or(b1, n1); }
+        r0 = row_or(r0, n0);
+        f0 = n0;
+        if (m3 == 1) a0 = row_or(a0, n0);
+        if (m3 == 2) b0 = row_or(b0, n0);
         const Row h0 = row_and(n0, mv0), h1 = row_and(n1, mv1);
-        for (uint64_t hit = ballot(row_any(h0) || row_any(h1)); hit; hit &= hit - 1) {
-            const int l = __ffsll((unsigned long long)hit) - 1;
-            const Row g = my >= 64 ? row_lane(h1, l) : row_lane(h0, l);
-            const uint32_t w = mword == 0 ? g.a : mword == 1 ? g.b : g.c;
-            if (mover && (my & 63) == l && (w & mbit)) x.mlay = layer;
+        uint64_t hit = ballot(row_any(h0) || row_any(h1));
+        if (hit) {
+            for (; hit; hit &= hit - 1) {
+                const int l = __ffsll((unsigned long long)hit) - 1;
+                const Row g = my >= 64 ? row_lane(h1, l) : row_lane(h0, l);
+                const uint32_t w = mword == 0 ? g.a : mword == 1 ? g.b : g.c;
+                if (mover && (my & 63) == l && (w & mbit)) x.mlay = layer;
+            }
+            // only a layer that reached a mover can have reached the last one
+            if (stop == (1 << 30) && !ballot(row_any(row_andn(mv0, r0)) || row_any(row_andn(mv1, r1)))) stop = layer + margin;
         }
-        if (stop == (1 << 30) && !ballot(row_any(row_andn(mv0, r0)) || row_any(row_andn(mv1, r1)))) stop = layer + margin;
         if (layer >= stop) break;
     }
     x.lastl = last;

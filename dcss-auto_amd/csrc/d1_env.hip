@@ -68,30 +68,41 @@ __host__ __device__ constexpr int state_bytes(int m) {
 // rejection with the v1 HP table gpu-d1/src/learn.cu:305-314, then three stairs by
 // reservoir choice from a copy of the RNG, then the initial reveal without reward).
 // roster_mode 1 and awake_pct draw after the energy draw.
+// A reset is one world's serial chain, and in small batches the launch lasts as long as the
+// slowest world: the spawnable cells and the stairs' eligible cells stay in registers (a cell is
+// selected by a ballot and scalar bit counts), a placed monster is found by a ballot over the
+// lanes' cells. Through LDS (prefix counts, binary searches, the occupancy bitmap set and read
+// cell by cell) and with the reservoirs filling the draw buffer, a reset with 8 monsters took
+// 27 us and one with 24 about 47, 5 to 8 times a plain step.
 __device__ __forceinline__ void reset(Ctx &x, const uint32_t *cells_g) {
     Smem *sm = x.sm;
     const D1Config *c = x.c;
-    for (int w = x.lane; w < ROWS_WORDS; w += 64) { sm->occ[w] = 0; sm->front[w] = cells_g[w]; sm->viewed[w] = 0; }
+    const bool has1 = x.lane < H - 64;
+    const Row zero{0, 0, 0};
+    const Row c0 = row_ld(cells_g, x.lane), c1 = has1 ? row_ld(cells_g, 64 + x.lane) : zero;
+    for (int w = x.lane; w < ROWS_WORDS; w += 64) { sm->occ[w] = 0; sm->viewed[w] = 0; }
     x.vlo = 0, x.vhi = H - 1;
     __syncthreads();
-    x.ncells = row_prefix(x, sm->front);
-    x.player = select_cell(x, sm->front, x.g.r(x.ncells));
+    const Rows cells = rows_count(c0, c1);
+    x.ncells = cells.total;
+    x.player = rows_select(cells, x.g.r(x.ncells));
     x.hp = c->hp; x.regen = 0; x.blocks = 0;
     x.ticks = 0; x.decisions = 0; x.killed = 0; x.floor_seen = 0;
     int mpos = -1, mhp = 0, men = -30000, mawake = 0, mkind = 0;
+#pragma unroll 1
     for (int i = 0; i < c->count; i++) {
+        auto taken = [&](int p) { return p == x.player || ballot(mpos == p); };   // only lanes < i hold a cell
         int p = 0, tries = 0;
         do {
-            p = select_cell(x, sm->front, x.g.r(x.ncells));
+            p = rows_select(cells, x.g.r(x.ncells));
             tries++;
-        } while ((p == x.player || bit(sm->occ, p)) && tries < 65536);
-        if (p == x.player || bit(sm->occ, p)) {   // unreachable in practice; first free cell
+        } while (taken(p) && tries < 65536);
+        if (taken(p)) {   // unreachable in practice; first free cell
             for (int j = 0; j < x.ncells; j++) {
-                p = select_cell(x, sm->front, j);
-                if (p != x.player && !bit(sm->occ, p)) break;
+                p = rows_select(cells, j);
+                if (!taken(p)) break;
             }
         }
-        occ_set(x, p, true);
         int kind = i % 6, hpv = 0;
         if (c->roster_mode == 0) { const int MHP[6] = {8, 10, 12, 16, 12, 10}; hpv = MHP[i % 6]; }
         int en = 70 + x.g.r(10);
@@ -100,33 +111,34 @@ __device__ __forceinline__ void reset(Ctx &x, const uint32_t *cells_g) {
         if (x.lane == i) { mpos = p; mhp = hpv; men = en; mawake = aw; mkind = kind; }
     }
     x.mpos = mpos; x.mhp = mhp; x.menergy = men; x.mawake = mawake; x.mkind = mkind;
+    if (x.lane < c->count) occ_set_lane(x, mpos);
+    __syncthreads();
     // Stairs: a copy of the RNG, reservoir over eligible cells in cell order.
     Rng s = x.g;
     x.first_stair_tick = -1;
     x.stairs = pack_stairs(-1, -1, -1);
-    int px = x.player % W, py = x.player / W;
+    const int px = x.player % W, py = x.player / W;
+    const Row o0 = row_andn(c0, row_ld(sm->occ, x.lane)), o1 = has1 ? row_andn(c1, row_ld(sm->occ, 64 + x.lane)) : zero;
+#pragma unroll 1
     for (int k = 0; k < 3; k++) {
         if (k >= c->stairs) break;
-        // eligible rows into sm->reach: cells & ~occ & cheb(player) >= 12 & cheb(prev stairs) >= 8
-        for (int y = x.lane; y < H; y += 64) {
-            Row e = row_andn(row_ld(sm->front, y), row_ld(sm->occ, y));
+        // eligible rows: cells & ~occ & cheb(player) >= 12 & cheb(prev stairs) >= 8
+        auto eligible = [&](Row e, int y) {
             if (iabs(y - py) < 12) e = row_andn(e, row_range(px - 11, px + 11));
             for (int q = 0; q < k; q++) {
                 int sp = stair_at(x, q);
                 if (iabs(y - sp / W) < 8) e = row_andn(e, row_range(sp % W - 7, sp % W + 7));
             }
-            row_st(sm->reach, y, e);
-        }
-        __syncthreads();
-        int total = row_prefix(x, sm->reach);
-        int chosen = reservoir(s, total, x.lane);
-        int sel = chosen >= 0 ? select_cell(x, sm->reach, chosen) : -1;
+            return e;
+        };
+        const Rows el = rows_count(eligible(o0, x.lane), eligible(o1, 64 + x.lane));
+        const int chosen = reservoir(s, el.total, x.lane);
+        const int sel = chosen >= 0 ? rows_select(el, chosen) : -1;
         x.stairs = (x.stairs & ~(0xFFFFULL << (16 * k))) | (uint64_t)(uint16_t)sel << (16 * k);
-        __syncthreads();
     }
     reveal(x);
     x.ftag = -1;   // a new player cell and new monster cells: the memo no longer applies
-    x.fld = -1;    // and the reach bitmap held the stairs' eligible cells
+    x.fld = -1;
     x.mrad = 0;    // nor does any stuck answer
 }
 
