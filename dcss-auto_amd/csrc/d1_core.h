@@ -912,6 +912,10 @@ __device__ __forceinline__ Row dilate(Row f, Row up, Row dn) {
     Row v = row_or(f, row_or(up, dn));
     return row_or(v, row_or(row_shl1(v), row_shr1(v)));
 }
+template <int V>
+struct Const {
+    static constexpr int value = V;
+};
 __device__ __forceinline__ void bfs(Ctx &x, uint64_t movers, int margin) {
     Smem *sm = x.sm;
     const int lane = x.lane;
@@ -939,50 +943,53 @@ __device__ __forceinline__ void bfs(Ctx &x, uint64_t movers, int margin) {
     const int my = mover ? x.mpos / W : 0, mword = mover ? (x.mpos % W) >> 5 : 0;
     const uint32_t mbit = mover ? 1u << ((x.mpos % W) & 31) : 0u;
     x.mlay = FAR;
-    int m3 = 0, stop = 1 << 30, last = 0;
-    // lanes with frontier cells in their first and second row: the second set is worked on only
-    // while the frontier is in or next to rows 64.. (lane 0 and lane 63 read zero rows past the
-    // wave's ends, and lane 6's second row is empty, so the map's edges need no masks)
-    uint64_t on0 = ballot(row_any(f0)), on1 = ballot(row_any(f1));
-    for (int layer = 1; layer < N; layer++) {
-        m3 = m3 == 2 ? 0 : m3 + 1;
-        Row n0, n1 = zero;
-        if ((on0 >> 63) | on1) {
+    int stop = 1 << 30, layer = 0;
+    // Whether the frontier is in or next to rows 64..: the second row set is worked on only then.
+    // (Lane 0 and lane 63 read zero rows past the wave's ends, and lane 6's second row is empty,
+    // so the map's edges need no masks.)
+    bool low = py >= 63;
+    // One layer; M3 = layer mod 3, a constant of each copy (the planes it feeds are then fixed).
+    // Returns true when the field is done.
+    auto step = [&](auto mod) {
+        constexpr int M3 = decltype(mod)::value;
+        Row n0 = dilate(f0, row_up(f0), row_dn(f0)), h1 = zero;
+        uint64_t on1 = 0;
+        if (low) {
             const Row f1_0 = row_lane(f1, 0), f0_63 = row_lane(f0, 63);
-            const Row u0 = row_up(f0), d0 = row_sel(lane == 63, f1_0, row_dn(f0));
-            const Row u1 = row_sel(lane == 0, f0_63, row_up(f1)), d1 = row_dn(f1);
-            n0 = row_andn(row_and(dilate(f0, u0, d0), fl0), r0);
-            n1 = row_andn(row_and(dilate(f1, u1, d1), fl1), r1);   // fl1 is zero in lanes 6..
-            r1 = row_or(r1, n1);
-            f1 = n1;
-            if (m3 == 1) a1 = row_or(a1, n1);
-            if (m3 == 2) b1 = row_or(b1, n1);
-            on1 = ballot(row_any(n1));
-        } else {
-            n0 = row_andn(row_and(dilate(f0, row_up(f0), row_dn(f0)), fl0), r0);
+            n0 = row_or(n0, row_sel(lane == 63, dilate(f1_0, zero, zero), zero));
+            const Row u1 = row_sel(lane == 0, f0_63, row_up(f1));
+            f1 = row_andn(row_and(dilate(f1, u1, row_dn(f1)), fl1), r1);   // fl1 is zero in lanes 6..
+            r1 = row_or(r1, f1);
+            if (M3 == 1) a1 = row_or(a1, f1);
+            if (M3 == 2) b1 = row_or(b1, f1);
+            h1 = row_and(f1, mv1);
+            on1 = ballot(row_any(f1));
         }
-        on0 = ballot(row_any(n0));
-        if (!(on0 | on1)) break;
-        last = layer;
-        r0 = row_or(r0, n0);
-        f0 = n0;
-        if (m3 == 1) a0 = row_or(a0, n0);
-        if (m3 == 2) b0 = row_or(b0, n0);
-        const Row h0 = row_and(n0, mv0), h1 = row_and(n1, mv1);
-        uint64_t hit = ballot(row_any(h0) || row_any(h1));
+        f0 = row_andn(row_and(n0, fl0), r0);
+        const uint64_t on0 = ballot(row_any(f0));
+        if (!(on0 | on1)) return true;
+        low = (on0 >> 63) | on1;
+        layer++;
+        r0 = row_or(r0, f0);
+        if (M3 == 1) a0 = row_or(a0, f0);
+        if (M3 == 2) b0 = row_or(b0, f0);
+        const Row h0 = row_and(f0, mv0);
+        uint64_t hit = ballot(row_any(row_or(h0, h1)));
         if (hit) {
             for (; hit; hit &= hit - 1) {
                 const int l = __ffsll((unsigned long long)hit) - 1;
-                const Row g = my >= 64 ? row_lane(h1, l) : row_lane(h0, l);
+                const Row g0 = row_lane(h0, l), g1 = row_lane(h1, l);
+                const Row g = row_sel(my >= 64, g1, g0);
                 const uint32_t w = mword == 0 ? g.a : mword == 1 ? g.b : g.c;
                 if (mover && (my & 63) == l && (w & mbit)) x.mlay = layer;
             }
             // only a layer that reached a mover can have reached the last one
-            if (stop == (1 << 30) && !ballot(row_any(row_andn(mv0, r0)) || row_any(row_andn(mv1, r1)))) stop = layer + margin;
+            if (stop == (1 << 30) && !ballot(row_any(row_or(row_andn(mv0, r0), row_andn(mv1, r1))))) stop = layer + margin;
         }
-        if (layer >= stop) break;
-    }
-    x.lastl = last;
+        return layer >= stop;
+    };
+    while (!step(Const<1>{}) && !step(Const<2>{}) && !step(Const<0>{})) {}   // a layer adds a cell: at most N
+    x.lastl = layer;
     row_st(sm->reach, lane, r0);
     row_st(sm->lay0, lane, a0);
     row_st(sm->lay1, lane, b0);

@@ -239,7 +239,7 @@ __device__ __forceinline__ bool primitive(Ctx &x, int d, float *out8, bool &saw,
         x.menergy = (int16_t)x.menergy;
         uint64_t movers = ballot(mine && x.mhp > 0 && x.mawake && x.menergy >= 80 && cheb_u(x.mpos, x.player) > 1);
         if (movers) {
-            if (x.fcache) field_memo(x);
+            if (x.stuck_cache) field_memo(x);   // the crowded build (a constant): the other holds no memo code
             else {
                 int maxspeed = 0;
                 for (int k = 0; k < 6; k++) maxspeed = imax(maxspeed, c->kinds[k].speed);
@@ -417,7 +417,7 @@ __device__ __forceinline__ uint32_t state_hash(Ctx &x) {
 }
 
 // ---------------------------------------------------------------- load / store
-__device__ __forceinline__ void store_world(Ctx &x, uint8_t *row, int max_m) {
+__device__ __forceinline__ void store_world(Ctx &x, uint8_t *row, int max_m, bool memo) {
     if (x.lane == 0) {
         Hdr h;
         h.rng_state = x.g.mode == 0 ? x.g.pcg_state() : ((uint64_t)x.g.key1 << 32 | x.g.key0);
@@ -443,7 +443,7 @@ __device__ __forceinline__ void store_world(Ctx &x, uint8_t *row, int max_m) {
     // every row after a reset, none when the player did not move
     uint32_t *vg = (uint32_t *)(row + off_viewed(max_m));
     for (int w = RW * x.vlo + x.lane; w < RW * (x.vhi + 1); w += 64) vg[w] = x.sm->viewed[w];
-    if (has_fcache(max_m)) {   // memo head: its player cell, last layer, the monsters' layers
+    if (memo) {   // memo head: its player cell, last layer, the monsters' layers
         uint32_t *fc = (uint32_t *)(row + off_fcache(max_m));
         if (x.lane == 0) { fc[0] = (uint32_t)x.ftag; fc[1] = (uint32_t)x.lastl | (uint32_t)x.rfloor << 31; }
         if (x.lane < max_m) {
@@ -513,7 +513,7 @@ struct Pre {
     int act;   // the action's low 32 bits
     int on;
 };
-__device__ __forceinline__ void prefetch_world(Pre &pf, const uint8_t *row, int max_m, const int64_t *actions,
+__device__ __forceinline__ void prefetch_world(Pre &pf, const uint8_t *row, int max_m, bool memo, const int64_t *actions,
                                                const uint8_t *active, int env, int lane) {
     pf.hv = ((const uint32_t *)row)[imin(lane, 23)];
     pf.mon = ((const u32x2 *)(row + OFF_MON))[imin(lane, max_m - 1)];
@@ -524,7 +524,7 @@ __device__ __forceinline__ void prefetch_world(Pre &pf, const uint8_t *row, int 
         pf.vw[i] = vg[w];
         pf.fl[i] = fg[w];
     }
-    pf.fh = has_fcache(max_m) ? ((const uint32_t *)(row + off_fcache(max_m)))[imin(lane, FC_HEAD - 1)] : 0u;
+    pf.fh = memo ? ((const uint32_t *)(row + off_fcache(max_m)))[imin(lane, FC_HEAD - 1)] : 0u;
     pf.act = ((const int *)actions)[2 * (size_t)env];   // little-endian: the int64's low half
     pf.on = active ? active[env] : 1;
 }
@@ -552,7 +552,7 @@ __device__ __forceinline__ void unpack_world(Ctx &x, const Pre &pf, int max_m) {
     }
     x.fld = -1;
     x.vlo = H, x.vhi = -1;   // no viewed row changed yet
-    if (has_fcache(max_m)) {
+    if (x.stuck_cache) {
         x.ftag = (int)__builtin_amdgcn_readlane((int)pf.fh, 0);
         const uint32_t h1 = (uint32_t)__builtin_amdgcn_readlane((int)pf.fh, 1);
         x.lastl = (int)(h1 & 0x7FFFFFFFu);
@@ -614,7 +614,7 @@ __global__ __launch_bounds__(64) void k_init(uint8_t *state, int n, int max_m, s
     x.decisions = 0; x.floor_seen = 0;
     x.mlay = FAR; x.lastl = 0;
     reset(x, cg);
-    store_world(x, row, max_m);
+    store_world(x, row, max_m, has_fcache(max_m));
     if (obs) write_obs(x, obs + (size_t)env * D1_OBS_BYTES);
     if (hash) {   // the digest costs about a tenth of a step: callers that do not ask skip it
         const uint32_t h = state_hash(x);
@@ -664,7 +664,7 @@ __device__ __forceinline__ void step_worlds(Smem &sm, uint8_t *state, int n, int
         asm volatile("" : "+v"(lane));
         x.lane = lane;
         uint8_t *row = state + (size_t)env * row_bytes;
-        prefetch_world(pf, row, max_m, actions, active, env, x.lane);
+        prefetch_world(pf, row, max_m, CROWD, actions, active, env, x.lane);
         const int on = __builtin_amdgcn_readfirstlane(pf.on);
         // the int64 action's low 32 bits as a signed int, as the reference's int parameter
         // takes it (gpu-d1/branches/d1-stairs-v2/src/learn.cu:853,904); values outside the
@@ -672,12 +672,13 @@ __device__ __forceinline__ void step_worlds(Smem &sm, uint8_t *state, int n, int
         const int action = __builtin_amdgcn_readfirstlane(pf.act);
         if (!on) continue;   // an inactive env keeps its state and all its output rows
         unpack_world<RM>(x, pf, max_m);
-        x.fcache = has_fcache(max_m) ? (uint32_t *)(row + off_fcache(max_m)) : nullptr;
+        // k_step runs layouts without the memo (has_fcache) only, k_step_crowd only those with it
+        x.fcache = CROWD ? (uint32_t *)(row + off_fcache(max_m)) : nullptr;
         const uint32_t *cg = (const uint32_t *)(row + off_cells(max_m));
         float o8[8];
         transition(x, action, o8, cg);
         x.t++;
-        store_world(x, row, max_m);
+        store_world(x, row, max_m, CROWD);
         if (out && x.lane == 0) {
             float4 *o4 = (float4 *)(out + (size_t)env * D1_OUT);
             o4[0] = make_float4(o8[0], o8[1], o8[2], o8[3]);
