@@ -47,6 +47,7 @@ def load():
             getattr(L, name).argtypes = []
         L.d1_init.argtypes = [p, i, i, p, p, C.c_uint64, p, p, p]
         L.d1_step.argtypes = [p, i, i, p, p, p, p, p, p, p, p]
+        L.d1_step_into.argtypes = [p, i, i, p, p, p, p, p, p, p, p, p]
         L.d1_heuristic.argtypes = [p, i, i, p, i, p, p]
         L.d1_sample.argtypes = [p, i, i, i, C.c_uint64, C.c_uint32, p, p, p]
         L.d1_sample_dev.argtypes = [p, i, i, i, C.c_uint64, p, C.c_uint32, p, p, p]

@@ -22,6 +22,7 @@
 #include "../../include/d1hip.h"
 
 #include "d1_core.h"
+#include "d1_internal.h"
 
 namespace d1 {
 
@@ -642,7 +643,8 @@ __host__ __device__ inline int step_blocks(int n, int wpb, int tail) {
 template <int RM, int WPB, bool CROWD>
 __device__ __forceinline__ void step_worlds(Smem &sm, uint8_t *state, int n, int max_m, size_t row_bytes,
                                             const D1Config *cfgp, const D1Tables &tab, const int64_t *actions,
-                                            uint8_t *obs, float *out, uint32_t *hash, const uint8_t *active) {
+                                            uint8_t *obs, float *out, uint32_t *hash, const uint8_t *active,
+                                            float *reward, uint8_t *done) {
     constexpr int TAIL = CROWD ? CROWD_TAIL : STEP_TAIL;
     const int g = step_groups(n, WPB, TAIL), blk = (int)blockIdx.x;   // first < n for every block of step_blocks
     const int first = blk < g ? WPB * blk : WPB * g + (blk - g), last = imin(n, blk < g ? first + WPB : first + 1);
@@ -684,6 +686,10 @@ __device__ __forceinline__ void step_worlds(Smem &sm, uint8_t *state, int n, int
             o4[0] = make_float4(o8[0], o8[1], o8[2], o8[3]);
             o4[1] = make_float4(o8[4], o8[5], o8[6], o8[7]);
         }
+        if (reward && x.lane == 0) {   // a rollout buffer's own columns (two copy launches a step)
+            reward[env] = o8[0];
+            done[env] = (uint8_t)o8[1];
+        }
         if (obs) write_obs(x, obs + (size_t)env * D1_OBS_BYTES);
         if (hash) {   // the digest costs about a tenth of a step: callers that do not ask skip it
             const uint32_t h = state_hash(x);
@@ -704,19 +710,21 @@ __device__ __forceinline__ void step_worlds(Smem &sm, uint8_t *state, int n, int
 template <int RM>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_step(
     uint8_t *state, int n, int max_m, size_t row_bytes, D1Config cfg, D1Tables tab, const int64_t *actions,
-    uint8_t *obs, float *out, uint32_t *hash, const uint8_t *active) {
+    uint8_t *obs, float *out, uint32_t *hash, const uint8_t *active, float *reward, uint8_t *done) {
     __shared__ Smem sm;
     __shared__ D1Config lcfg;
     for (int i = lane_id(); i < (int)(sizeof(D1Config) / 4); i += 64) ((uint32_t *)&lcfg)[i] = ((const uint32_t *)&cfg)[i];
     __syncthreads();
-    step_worlds<RM, STEP_WPB, false>(sm, state, n, max_m, row_bytes, &lcfg, tab, actions, obs, out, hash, active);
+    step_worlds<RM, STEP_WPB, false>(sm, state, n, max_m, row_bytes, &lcfg, tab, actions, obs, out, hash, active,
+                                     reward, done);
 }
 template <int RM>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_step_crowd(
     uint8_t *state, int n, int max_m, size_t row_bytes, D1Config cfg, D1Tables tab, const int64_t *actions,
-    uint8_t *obs, float *out, uint32_t *hash, const uint8_t *active) {
+    uint8_t *obs, float *out, uint32_t *hash, const uint8_t *active, float *reward, uint8_t *done) {
     __shared__ Smem sm;
-    step_worlds<RM, CROWD_WPB, true>(sm, state, n, max_m, row_bytes, &cfg, tab, actions, obs, out, hash, active);
+    step_worlds<RM, CROWD_WPB, true>(sm, state, n, max_m, row_bytes, &cfg, tab, actions, obs, out, hash, active,
+                                     reward, done);
 }
 
 // ---------------------------------------------------------------- monster-wait workload
@@ -1101,8 +1109,9 @@ int d1_heuristic(const void *state, int n, int max_monsters, const D1Config *cfg
                        max_monsters, (size_t)d1::state_bytes(max_monsters), cfg->count, joint, actions);
     return (int)hipGetLastError();
 }
-int d1_step(void *state, int n, int max_monsters, const D1Config *cfg, const D1Tables *tab, const int64_t *actions,
-            uint8_t *obs, float *out, uint32_t *hash, const uint8_t *active, void *stream) {
+static int launch_step(void *state, int n, int max_monsters, const D1Config *cfg, const D1Tables *tab, const int64_t *actions,
+                       uint8_t *obs, float *out, uint32_t *hash, const uint8_t *active, float *reward, uint8_t *done,
+                       void *stream) {
     int e = d1::validate(n, max_monsters, cfg, tab);
     if (e) return e;
     if (!state || !actions) return D1_E_ARG;
@@ -1113,7 +1122,16 @@ int d1_step(void *state, int n, int max_monsters, const D1Config *cfg, const D1T
     const int tail = max_monsters > 8 ? d1::CROWD_TAIL : d1::STEP_TAIL;
     hipLaunchKernelGGL(kern, dim3(d1::step_blocks(n, wpb, tail)), dim3(64), 0, (hipStream_t)stream,
                        (uint8_t *)state, n, max_monsters,
-                       (size_t)d1::state_bytes(max_monsters), *cfg, *tab, actions, obs, out, hash, active);
+                       (size_t)d1::state_bytes(max_monsters), *cfg, *tab, actions, obs, out, hash, active, reward, done);
     return (int)hipGetLastError();
+}
+int d1_step(void *state, int n, int max_monsters, const D1Config *cfg, const D1Tables *tab, const int64_t *actions,
+            uint8_t *obs, float *out, uint32_t *hash, const uint8_t *active, void *stream) {
+    return launch_step(state, n, max_monsters, cfg, tab, actions, obs, out, hash, active, nullptr, nullptr, stream);
+}
+int d1_step_into(void *state, int n, int max_monsters, const D1Config *cfg, const D1Tables *tab, const int64_t *actions,
+                 uint8_t *obs, float *out, uint32_t *hash, float *reward, uint8_t *done, void *stream) {
+    if (n && (!reward || !done)) return D1_E_ARG;
+    return launch_step(state, n, max_monsters, cfg, tab, actions, obs, out, hash, nullptr, reward, done, stream);
 }
 }

@@ -150,6 +150,20 @@ class Env:
                                     None, None, self.stream), 'd1_step')
         return self.obs[lo:hi], self.out[lo:hi]
 
+    def step_into(self, actions, obs, reward, done):
+        """step() of every world into a rollout buffer's rows: the observation into `obs` (as
+        step()'s obs), the reward and done columns of `out` into `reward` (fp32 [batch]) and
+        `done` (uint8 [batch]) by the same launch."""
+        for t, dt, numel in ((actions, torch.int64, self.batch), (obs, torch.uint8, self.batch * 1800),
+                             (reward, torch.float32, self.batch), (done, torch.uint8, self.batch)):
+            if not (t.device == self.device and t.dtype == dt and t.is_contiguous() and t.numel() == numel):
+                raise ValueError('step_into takes contiguous int64 actions, uint8 obs, float32 reward and uint8 done '
+                                 'buffers of the batch on the env device')
+        _lib.check(self.lib.d1_step_into(self.state.data_ptr(), self.batch, self.max_monsters, C.byref(self.cfg),
+                                         C.byref(self.tables), actions.data_ptr(), obs.data_ptr(), self.out.data_ptr(),
+                                         self.hash.data_ptr() if self.with_hash else None, reward.data_ptr(),
+                                         done.data_ptr(), self.stream), 'd1_step_into')
+
     def step(self, actions, active=None, obs=None):
         """`obs` optionally redirects this step's observation into another uint8
         [batch, 15, 15, 8]-shaped buffer (e.g. a rollout-buffer slice); self.obs then

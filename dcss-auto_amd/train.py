@@ -5,7 +5,7 @@ One update = a T-step rollout (policy forward from the uint8 observation with th
 counter-RNG sample in the same kernel, env step; each writes straight into the rollout
 buffer) followed by FastPPO.update (GAE, advantage normalisation, epochs of shuffled
 minibatches). With
-graph=True the whole rollout — T x (forward + sample, step, reward/done copies), the
+graph=True the whole rollout — T x (forward + sample, step), the
 bootstrap value and the step-counter advance — is captured once in a HIP graph and
 replayed; the sampler reads its counter step from the device, so every replay draws new
 actions.
@@ -28,6 +28,7 @@ import torch
 from . import _lib
 from . import policy as P
 from . import ppo as ppo_mod
+from .env import Env
 
 # Checkpoint layout version: 2 added the trainer-settings record and grew crowded env state
 # rows (more than 8 monsters) by the 2,656-byte distance-field memo; 3 added the monsters'
@@ -79,14 +80,20 @@ class Trainer:
     def _rollout_body(self):
         buf, env = self.buf, self.env
         b1, b2, b3 = self.bias
+        # the step writes the reward and done rows itself (two copy launches a step), unless the
+        # environment has a step() of its own
+        plain = type(env) is Env and 'step' not in vars(env)
         buf.obs[0].copy_(self.next_obs)
         for k in range(self.T):   # forward + sample in one kernel, the counter step read on the device
             P.policy_fwd_sample(buf.obs[k], self.wpk, b1, b2, b3, self.seed, k, buf.actions[k], buf.logp[k],
                                 buf.values[k], t_dev=self.t_dev)
             dst = buf.obs[k + 1] if k + 1 < self.T else self.next_obs
-            env.step(buf.actions[k], obs=dst)
-            buf.rewards[k].copy_(env.out[:, 0])
-            buf.dones[k].copy_(env.out[:, 1])
+            if plain:
+                env.step_into(buf.actions[k], dst, buf.rewards[k], buf.dones[k])
+            else:
+                env.step(buf.actions[k], obs=dst)
+                buf.rewards[k].copy_(env.out[:, 0])
+                buf.dones[k].copy_(env.out[:, 1])
         P.policy_fwd(self.next_obs, self.wpk, b1, b2, b3, logits=self.logits, value=buf.bootstrap)
         self.t_dev.add_(self.T)
 
