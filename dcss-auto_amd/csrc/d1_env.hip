@@ -623,18 +623,17 @@ __global__ __launch_bounds__(64) void k_init(uint8_t *state, int n, int max_m, s
     }
 }
 
-// Worlds per k_step workgroup: WPB consecutive worlds (each next world's loads overlap the
-// current one's stores and observation, so only a group's first load waits), except the
-// last STEP_TAIL worlds, one per workgroup: the workgroups dispatched last then hold one
-// world, which shortens the tail in which a few slow worlds (resets, long monster turns)
-// run on an otherwise idle chip (k_step 193 -> 187 us at 65,536 worlds). WPB is 4 for the
-// <= 8 monster build (0.176 -> 0.171 ms at 65,536 worlds) and 3 for the crowded build
-// (C5 k_step: 2 worlds 3.38 ms, 3 worlds 3.35, 4 worlds 3.37). The <= 8 monster build's tail
-// is 4,096 worlds: the C3 rollout steps its 65,536 worlds as two ranges of 32,768 on two
-// streams, where the other range's kernels fill the idle CUs (rollout 364.7 -> 375.7 M
-// decisions/s against a tail of 8,192; 0: 368.2, 2,048: 374.3); the crowded build keeps 8,192
-// (C5 k_step 2.063 ms against 2.090 with 4,096).
-constexpr int STEP_TAIL = 4096, CROWD_TAIL = 8192, STEP_WPB = 4, CROWD_WPB = 3;
+// Worlds per k_step workgroup: WPB consecutive worlds, except the last TAIL worlds, one per
+// workgroup: those dispatched last then hold one world, which shortens the end of the launch, in
+// which a few slow worlds (resets, long monster turns) run on an otherwise idle chip. Fewer
+// worlds a workgroup balance better, but each workgroup pays its start (and k_step the copy of
+// its configuration to LDS). With resets a third of what they were, at 65,536 / 32,768 / 8,192
+// worlds of 8 monsters: 4 worlds and a tail of 4,096 (at 5 waves per SIMD) 119.7 / 75.1 / 44.5
+// us, 2 worlds and a tail of 8,192 (at 6 waves) 107.8 / 65.7 / 33.1; 2 and 4,096 110.0 / 66.0 /
+// 33.6, 3 and 8,192 108.2 / 65.4 / 33.5, one world each 118.9 / 69.2. Crowded build, 262,144 and
+// 32,768 worlds of 40, 16,384 of 24: 3 worlds and a tail of 8,192 2,329 / 396 / 80.3 us, of
+// 16,384 2,326 / 385 / 69.1, of 32,768 2,322 / 386 / 68.9.
+constexpr int STEP_TAIL = 8192, CROWD_TAIL = 16384, STEP_WPB = 2, CROWD_WPB = 3;
 __host__ __device__ inline int step_groups(int n, int wpb, int tail) { return (n - (n < tail ? n : tail)) / wpb; }
 __host__ __device__ inline int step_blocks(int n, int wpb, int tail) {
     const int g = step_groups(n, wpb, tail);
@@ -656,7 +655,7 @@ __device__ __forceinline__ void step_worlds(Smem &sm, uint8_t *state, int n, int
     // current one stores its state and observation held 12 more registers across those
     // phases: at 4 waves per SIMD it paid (0.176 -> 0.171 ms at C3), but with the lane
     // masks no longer held through the monster loop both builds run more waves per SIMD
-    // without it, whose latency hiding does more (C3 k_step 0.152 -> 0.140 ms at 5 waves;
+    // without it, whose latency hiding does more (C3 k_step 0.152 -> 0.140 ms at 5 waves then;
     // in the crowded build the held row had gone to scratch, about 7 KB of traffic a world).
     Pre pf;
     for (int env = first; env < last; env++) {
@@ -698,17 +697,17 @@ __device__ __forceinline__ void step_worlds(Smem &sm, uint8_t *state, int n, int
     }
 }
 
-// Two builds of the same step. A world with at most 8 monsters spends its time in straight
-// issue-bound code (observation, reveal, scalar rules): 4 waves per SIMD without spills. The
-// crowded layouts (up to 64 monsters) spend it in serial monster turns whose LDS and
-// cross-lane latencies want more waves in flight: 6 waves per SIMD, which costs some
-// register spills (measured at 262,144 worlds x 40 monsters: 8.3 -> 7.0 ms per step; at
-// 65,536 x 8 the same build is 0.17 -> 0.33 ms, hence two builds). The <= 8 monster build
-// reads its configuration from an LDS copy, which keeps the fields out of scalar registers
-// (190 -> 104 spilled to VGPR lanes; 0.171 -> 0.168 ms at 65,536 worlds); in the crowded
-// build the same copy costs 4.69 -> 5.19 ms, so it reads the kernel argument.
+// Two builds of the same step, both 6 waves per SIMD (80 VGPRs, none spilled). A world with at
+// most 8 monsters spends its time in straight issue-bound code (observation, reveal, scalar
+// rules); the crowded layouts (up to 64 monsters) spend it in serial monster turns, keep a
+// complete distance field in the row and the player view in LDS. (k_step at 65,536 worlds, same
+// world split: 4 and 5 waves 118.8 and 119.5 us, 6 waves 115.0, and with two worlds a workgroup 6
+// waves 110.0, 7 112.1; crowded at 262,144 x 40: 5 waves 2,524 us, 6 2,326, 7 2,356.) The <= 8
+// monster build reads its configuration from an LDS copy, which keeps the fields out of scalar
+// registers (190 -> 104 spilled to VGPR lanes; 0.171 -> 0.168 ms at 65,536 worlds); in the
+// crowded build the same copy costs 4.69 -> 5.19 ms, so it reads the kernel argument.
 template <int RM>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_step(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_step(
     uint8_t *state, int n, int max_m, size_t row_bytes, D1Config cfg, D1Tables tab, const int64_t *actions,
     uint8_t *obs, float *out, uint32_t *hash, const uint8_t *active, float *reward, uint8_t *done) {
     __shared__ Smem sm;
