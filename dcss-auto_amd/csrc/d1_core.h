@@ -294,6 +294,16 @@ struct Rng {
         }
         return next();
     }
+    // Passes over the next n draws.
+    __device__ __forceinline__ void skip(uint32_t n) {
+        o += n;
+        if (mode == 0)
+            while (o > 64u) {   // a fill happens at most 64 draws after the last one
+                const uint32_t rest = o - 64u;
+                fill(base + 64u);
+                o = rest;
+            }
+    }
     // PCG32 state before draw k (what the sequential generator would hold now)
     __device__ __forceinline__ uint64_t pcg_state() const {
         uint32_t j = base + o - sb;
@@ -416,6 +426,9 @@ struct Ctx {
     // clears it), so the next act draws its rotation and waits without searching.
     int mrad = 0;
     bool stuck_cache = false;
+    // This lane's monster had no walkable neighbour when the turn's acts began, and none has
+    // opened since (kept by the stuck_cache kernels within a turn only).
+    bool mblk = false;
     int lastl;   // last layer the field holds: a reached cell next to an unreached one is on it
     int lane;
     // distance-field memo in the state row (crowded layouts): its address, the player cell the
@@ -996,9 +1009,31 @@ __device__ __forceinline__ void bfs(Ctx &x, uint64_t movers, int margin) {
     if (has1) { row_st(sm->reach, 64 + lane, r1); row_st(sm->lay0, 64 + lane, a1); row_st(sm->lay1, 64 + lane, b1); }
     __syncthreads();
 }
-// Cells a and b changed occupancy: stuck answers whose search read either are dropped.
+// Cells a (freed) and b (taken, or a again) changed occupancy: stuck answers whose search read
+// either are dropped, and a monster next to the freed cell is no longer known to be shut in.
 __device__ __forceinline__ void stuck_touch(Ctx &x, int a, int b) {
-    if (x.mrad > 0 && (cheb_u(x.mpos, a) <= x.mrad || cheb_u(x.mpos, b) <= x.mrad)) x.mrad = 0;
+    const int da = cheb_u(x.mpos, a);
+    if (x.mrad > 0 && (da <= x.mrad || cheb_u(x.mpos, b) <= x.mrad)) x.mrad = 0;
+    x.mblk = x.mblk && da > 1;
+}
+// Whether this lane's monster, not next to the player, has no walkable neighbour: choose_move
+// then draws its rotation and waits. Three columns of three rows, as two words and a funnel
+// shift a row.
+__device__ __forceinline__ bool shut_in(const Ctx &x) {
+    const int mx = (int)((uint32_t)x.mpos % W), my = (int)((uint32_t)x.mpos / W);
+    const int k = (mx - 1) >> 5;
+    const uint32_t sh = (uint32_t)(mx - 1) & 31u;
+    uint32_t open = 0;
+#pragma unroll
+    for (int dy = -1; dy <= 1; dy++) {
+        const int y = my + dy;
+        if ((unsigned)y >= (unsigned)H) continue;
+        const int wl = y * RW + imax(k, 0), wh = y * RW + imin(k + 1, RW - 1);   // in the row either way
+        const uint32_t lo = k >= 0 ? x.sm->floor[wl] & ~x.sm->occ[wl] : 0u;
+        const uint32_t hi = k + 1 < RW ? x.sm->floor[wh] & ~x.sm->occ[wh] : 0u;
+        open |= __builtin_amdgcn_alignbit(hi, lo, sh);
+    }
+    return (open & 7u) == 0;   // the monster's own cell is occupied
 }
 // gpu-d1/src/sim.h:254-269
 // The mover's absolute layer follows it (the cell it steps to is a reached neighbour).
