@@ -169,6 +169,7 @@ __device__ __forceinline__ int reveal_learn(LCtx &c) {
         fresh = row_popc(row_and(chg, row_ld(sm->floor, y)));
         cnt = row_popc(chg);
     }
+    if (!ballot(cnt > 0)) return 0;   // every viewed cell was known: no anchor can change either
     int pre = cnt;   // inclusive prefix over view rows
     for (int o = 1; o < 16; o <<= 1) { int v = __shfl_up(pre, o); if (x.lane >= o) pre += v; }
     __syncthreads();
@@ -396,9 +397,10 @@ struct KB {
     int mlayer;          // this lane's monster layer
 };
 // Lane l keeps rows l and (l < 6) 64 + l of the frontier, reach, known floor and anchors in
-// registers; vertical neighbours arrive by lane shuffles, so a layer needs no LDS round
-// trip and no barrier. Reach, the layer planes, the last layer's frontier and the anchor
-// rows are published at the end.
+// registers, as bfs() does (its layers by constant mod 3, rows 64.. only while the frontier is
+// near them). What the search looks for is one set of cells: a layer that meets none of them can
+// neither finish the search nor give a layer, so only the others run the checks. Reach, the layer
+// planes and the anchor rows are published at the end.
 __device__ __forceinline__ uint32_t row_word(Row r, int w) { return w == 0 ? r.a : w == 1 ? r.b : r.c; }
 __device__ __forceinline__ KB known_bfs(LCtx &c, bool want_anchor, int want_stairs, bool want_monster) {
     Ctx &x = c.x;
@@ -416,33 +418,39 @@ __device__ __forceinline__ KB known_bfs(LCtx &c, bool want_anchor, int want_stai
         a0 = row_ld(L->anch, lane);
         if (has1) a1 = row_ld(L->anch, 64 + lane);
     }
+    Row w0 = a0, w1 = a1;   // the wanted cells
     const int py = x.player / W, px = x.player % W;
     const Row pbit = row_range(px, px);
     Row f0 = lane == py ? pbit : zero, f1 = has1 && 64 + lane == py ? pbit : zero;
     Row r0 = f0, r1 = f1;
     Row e0 = zero, e1 = zero, g0 = zero, g1 = zero;   // layer % 3 == 1, layer % 3 == 2
-    int m3 = 0;
     // wanted stairs: holder lane, register row and word of each (uniform)
     const int s0 = stair_at(x, 0), s1 = stair_at(x, 1), s2 = stair_at(x, 2);
+    auto want_cell = [&](int p) {
+        const int sy = p / W;
+        const Row bits = lane == (sy & 63) ? row_range(p % W, p % W) : zero;
+        if (sy >= 64) w1 = row_or(w1, bits);
+        else w0 = row_or(w0, bits);
+    };
+    if (want_stairs & 1) want_cell(s0);
+    if (want_stairs & 2) want_cell(s1);
+    if (want_stairs & 4) want_cell(s2);
     // this lane's monster cell, when it is wanted: holder lane and word of its row
     const bool mneed = want_monster && lane_alive(c) && in_view(x, x.mpos);
     const int my = mneed ? x.mpos / W : 0, mx = mneed ? x.mpos % W : 0;
     const int msrc = my & 63, mword = mx >> 5;
     const uint32_t mbit = 1u << (mx & 31);
-    for (int layer = 0; layer < N; layer++) {
-        if (layer > 0) {
-            const Row f1_0 = row_lane(f1, 0), f0_63 = row_lane(f0, 63);
-            const Row u0 = row_sel(lane == 0, zero, row_up(f0)), d0 = row_sel(lane == 63, f1_0, row_dn(f0));
-            const Row u1 = row_sel(lane == 0, f0_63, row_up(f1)), d1 = row_sel(lane >= H - 65, zero, row_dn(f1));
-            const Row n0 = row_andn(row_and(dilate(f0, u0, d0), k0), r0);
-            const Row n1 = has1 ? row_andn(row_and(dilate(f1, u1, d1), k1), r1) : zero;
-            r0 = row_or(r0, n0); r1 = row_or(r1, n1);
-            f0 = n0; f1 = n1;
-            m3 = m3 == 2 ? 0 : m3 + 1;
-            if (m3 == 1) { e0 = row_or(e0, n0); e1 = row_or(e1, n1); }
-            if (m3 == 2) { g0 = row_or(g0, n0); g1 = row_or(g1, n1); }
-            if (!ballot(row_any(n0) || row_any(n1))) break;
-        }
+    if (want_monster) {   // the cells as bit rows, through the frontier bitmap's space
+        row_st(sm->front, lane, zero);
+        if (has1) row_st(sm->front, 64 + lane, zero);
+        __syncthreads();
+        if (mneed) atomicOr(&sm->front[my * RW + mword], mbit);
+        __syncthreads();
+        w0 = row_or(w0, row_ld(sm->front, lane));
+        if (has1) w1 = row_or(w1, row_ld(sm->front, 64 + lane));
+    }
+    // the checks after a layer: true when nothing wanted is missing
+    auto check = [&](int layer) {
         bool done = true;
         if (want_anchor && r.alayer < 0) {
             const Row h0 = row_and(f0, a0), h1 = row_and(f1, a1);
@@ -473,14 +481,43 @@ __device__ __forceinline__ KB known_bfs(LCtx &c, bool want_anchor, int want_stai
                 if (ballot(mneed && r.mlayer < 0)) done = false;
             }
         }
-        if (done) break;
-    }
+        return done;
+    };
+    int layer = 0;
+    bool low = py >= 63;
+    // grows one layer (M3 = layer mod 3); true when the search is over
+    auto step = [&](auto mod) {
+        constexpr int M3 = decltype(mod)::value;
+        Row n0 = dilate(f0, row_up(f0), row_dn(f0));
+        uint64_t on1 = 0;
+        if (low) {
+            const Row f1_0 = row_lane(f1, 0), f0_63 = row_lane(f0, 63);
+            n0 = row_or(n0, row_sel(lane == 63, dilate(f1_0, zero, zero), zero));
+            const Row u1 = row_sel(lane == 0, f0_63, row_up(f1));
+            f1 = row_andn(row_and(dilate(f1, u1, row_dn(f1)), k1), r1);   // k1 is zero in lanes 6..
+            r1 = row_or(r1, f1);
+            if (M3 == 1) e1 = row_or(e1, f1);
+            if (M3 == 2) g1 = row_or(g1, f1);
+            on1 = ballot(row_any(f1));
+        }
+        f0 = row_andn(row_and(n0, k0), r0);
+        const uint64_t on0 = ballot(row_any(f0));
+        if (!(on0 | on1)) return true;
+        low = (on0 >> 63) | on1;
+        layer++;
+        r0 = row_or(r0, f0);
+        if (M3 == 1) e0 = row_or(e0, f0);
+        if (M3 == 2) g0 = row_or(g0, f0);
+        if (!ballot(row_any(row_or(row_and(f0, w0), row_and(f1, w1))))) return false;
+        return check(layer);
+    };
+    if (!check(0))
+        while (!step(Const<1>{}) && !step(Const<2>{}) && !step(Const<0>{})) {}   // a layer adds a cell: at most N
     row_st(sm->reach, lane, r0);
-    row_st(sm->front, lane, f0);
     row_st(sm->lay0, lane, e0);
     row_st(sm->lay1, lane, g0);
     if (has1) {
-        row_st(sm->reach, 64 + lane, r1); row_st(sm->front, 64 + lane, f1);
+        row_st(sm->reach, 64 + lane, r1);
         row_st(sm->lay0, 64 + lane, e1); row_st(sm->lay1, 64 + lane, g1);
     }
     if (want_anchor) {   // the nearest layer's anchors; none reachable: the set is not needed
@@ -552,6 +589,7 @@ __device__ __forceinline__ void primitive_learn(LCtx &c, int d, int limit, POut 
     Smem *sm = x.sm;
     const D1Config *cf = x.c;
     int milli = 0;
+    bool moved = false;
     x.blocks = 0;
     x.regen += cf->regen;
     while (x.regen >= 100) { x.hp = imin(cf->hp, x.hp + 1); x.regen -= 100; }
@@ -572,10 +610,12 @@ __device__ __forceinline__ void primitive_learn(LCtx &c, int d, int limit, POut 
                         x.killed++;
                     } else if (x.lane == id) x.mhp = nh;
                 }
-            } else x.player = p;
+            } else x.player = p, moved = true;
         }
     }
-    reveal_learn(c);   // EXPLORE_MILLI = 0, the reveal still updates memory
+    // EXPLORE_MILLI = 0, the reveal still updates memory; where the player stands was revealed by
+    // the move there or the reset, and the view depends on the cell alone
+    if (moved) reveal_learn(c);
     o.saw_awake = visible_awake(x);
     o.saw_enemy = visible_enemy(c);
     const bool clear = d == 18 && stair_index(x) > 0 && x.hp > 0;
