@@ -140,6 +140,13 @@ __device__ __forceinline__ int popc_below(Row r, int xx) {
     return __popc(r.a) + __popc(r.b) + __popc(r.c & ((1u << (xx - 64)) - 1u));
 }
 
+// columns x0 .. x0 + 16 of an 80-bit row (x0 from -8); columns outside the map read 0
+__device__ __forceinline__ uint32_t row_window17(Row r, int x0) {
+    if (x0 < 0) return (r.a << -x0) & 0x1FFFFu;
+    const int k = x0 >> 5;
+    const uint32_t lo = k == 0 ? r.a : k == 1 ? r.b : r.c, hi = k == 0 ? r.b : k == 1 ? r.c : 0u;
+    return __builtin_amdgcn_alignbit(hi, lo, (uint32_t)x0 & 31u) & 0x1FFFFu;
+}
 // reveal (learn.cu:298-336): mark the view, count fresh floor, then replay the
 // frontier refreshes in the reference's order.
 __device__ __forceinline__ int reveal_learn(LCtx &c) {
@@ -170,49 +177,67 @@ __device__ __forceinline__ int reveal_learn(LCtx &c) {
         cnt = row_popc(chg);
     }
     if (!ballot(cnt > 0)) return 0;   // every viewed cell was known: no anchor can change either
-    int pre = cnt;   // inclusive prefix over view rows
-    for (int o = 1; o < 16; o <<= 1) { int v = __shfl_up(pre, o); if (x.lane >= o) pre += v; }
-    __syncthreads();
-    if (mine) { row_st(sm->viewed, y, row_or(mask, old)); row_st(sm->front, y, chg); }
+    const int pre = wave_scan(cnt);   // inclusive prefix over view rows
+    // the newly viewed cells as 17-column window rows: rows 1..15 are the view's, 0 and 16 empty
+    if (x.lane < 15) sm->rq[x.lane + 1] = mine ? row_window17(chg, wx0) : 0u;
+    else if (x.lane < 17) sm->rq[16 * (x.lane - 15)] = 0u;
     if (x.lane < 15) L->cbase[x.lane] = pre - cnt;
     __syncthreads();
-    Row a1{0, 0, 0};
-    if (arow) a1 = anchor_row(sm, ya);
+    if (mine) row_st(sm->viewed, y, row_or(mask, old));
     __syncthreads();
-    if (arow) { row_st(sm->reach, ya, row_xor(a0, a1)); row_st(L->anch, ya, a1); }
+    const int total = (int)wave_sum((uint32_t)fresh);
+    x.floor_seen += total;
+    Row a1{0, 0, 0};
+    if (arow) {
+        a1 = anchor_row(sm, ya);
+        row_st(L->anch, ya, a1);
+    }
+    // the window cells that became or stopped being anchors, listed row by row (a lane of each
+    // row writes its own): there are a few tens of them, so the keys below take one pass
+    uint32_t diff = arow ? row_window17(row_xor(a0, a1), wx0) : 0u;
+    const int dcnt = __popc(diff), dpre = wave_scan(dcnt), changed = lane_val(dpre, 63);
+    if (!changed) {
+        __syncthreads();
+        return total;
+    }
+    uint16_t *cells = (uint16_t *)sm->lay0;   // dead between a step's searches
+    static_assert(WIN * WIN * 2 <= (int)sizeof(Smem::lay0), "the window's cells fit");
+    for (int o = dpre - dcnt; diff; diff &= diff - 1, o++) cells[o] = (uint16_t)(x.lane * WIN + __ffs(diff) - 1);
     // list positions of anchors inside the window
     for (int j = x.lane; j < c.nf; j += 64) {
         int p = c.lst[j], wx = p % W - wx0, wy = p / W - wy0;
         if (wx >= 0 && wx < WIN && wy >= 0 && wy < WIN) L->wslot[wy * WIN + wx] = (int16_t)j;
     }
     __syncthreads();
-    // key of each changed window cell: its first position in the refresh sequence
-    auto in_chg = [&](int qx, int qy) -> bool {
-        return qx >= px - 7 && qx <= px + 7 && qy >= py - 7 && qy <= py + 7 && inb(qx, qy) && bit_at(sm->front, qx, qy);
-    };
-    auto rank = [&](int qx, int qy) -> int {
-        return L->cbase[qy - (py - 7)] + popc_below(row_ld(sm->front, qy), qx);
-    };
-    int key[5];
-    int adds = 0;
+    // key of each changed window cell: its first position in the refresh sequence (newly viewed
+    // cell of rank k at 9 k, its neighbour in direction d at 9 k + 1 + d). A newly viewed cell at
+    // offset (ox, oy) has the changed cell as its neighbour in direction dir_of[oy + 1][ox + 1].
+    int key[5], cell[5];
 #pragma unroll
     for (int k = 0; k < 5; k++) {
-        int w = x.lane + 64 * k, qx = wx0 + w % WIN, qy = wy0 + w / WIN;
         key[k] = INF;
-        if (w < WIN * WIN && inb(qx, qy) && bit_at(sm->reach, qx, qy)) {
-            int kk = in_chg(qx, qy) ? 9 * rank(qx, qy) : INF;
+        cell[k] = 0;
+        const int j = x.lane + 64 * k;
+        if (64 * k < changed && j < changed) {
+            const int wc = cells[j], wy = (int)((uint32_t)wc / WIN), wx = wc - wy * WIN;
+            constexpr int dir_of[3][3] = {{5, 2, 6}, {1, -1, 3}, {4, 0, 7}};
+            int kk = INF;
 #pragma unroll
-            for (int d = 0; d < 8; d++) {
-                int ddx = d == 1 || d == 4 || d == 5 ? 1 : d == 3 || d == 6 || d == 7 ? -1 : 0;
-                int ddy = d == 0 || d == 4 || d == 7 ? -1 : d == 2 || d == 5 || d == 6 ? 1 : 0;
-                int cx = qx - ddx, cy = qy - ddy;   // q = neighbor(c, d)
-                if (in_chg(cx, cy)) kk = imin(kk, 9 * rank(cx, cy) + 1 + d);
+            for (int oy = -1; oy <= 1; oy++) {
+                const int r = wy + oy;
+                const uint32_t pat = (unsigned)r < (unsigned)WIN ? sm->rq[r] << 1 : 0u;   // bit column + 1
+                int rank = L->cbase[imin(imax(r - 1, 0), 14)] + __popc(pat & ((1u << wx) - 1u));
+#pragma unroll
+                for (int ox = 0; ox < 3; ox++) {
+                    const bool on = (pat >> (wx + ox)) & 1u;
+                    if (on) kk = imin(kk, 9 * rank + 1 + dir_of[oy + 1][ox]);
+                    rank += on;
+                }
             }
             key[k] = kk;
-            adds += bit_at(L->anch, qx, qy);
+            cell[k] = wc;
         }
     }
-    adds = (int)wave_sum((uint32_t)adds);
     uint16_t *lst = c.lst;
     int nf = c.nf;
     for (;;) {
@@ -220,8 +245,7 @@ __device__ __forceinline__ int reveal_learn(LCtx &c) {
         int m = wave_min(lm);
         if (m == INF) break;
         int wl = __ffsll((unsigned long long)ballot(lm == m)) - 1;
-        int wc = key[0] == m ? x.lane : key[1] == m ? x.lane + 64 : key[2] == m ? x.lane + 128
-               : key[3] == m ? x.lane + 192 : x.lane + 256;
+        int wc = key[0] == m ? cell[0] : key[1] == m ? cell[1] : key[2] == m ? cell[2] : key[3] == m ? cell[3] : cell[4];
         wc = lane_val(wc, wl);
         if (x.lane == wl) {
 #pragma unroll
@@ -247,8 +271,6 @@ __device__ __forceinline__ int reveal_learn(LCtx &c) {
     __threadfence_block();
     c.nf = nf;
     __syncthreads();
-    int total = (int)wave_sum((uint32_t)fresh);
-    x.floor_seen += total;
     return total;
 }
 
@@ -387,8 +409,8 @@ __device__ __forceinline__ void reset_learn(LCtx &c) {
 }
 
 // ---------------------------------------------------------------- known-floor BFS (learn.cu:222-266)
-// Bit-parallel BFS over viewed floor from the player into sm->reach and the layer-mod-3
-// planes sm->lay0/lay1. Stops when the first layer holding an anchor is found (its anchors then
+// Bit-parallel BFS over viewed floor from the player into the layer-mod-3 planes sm->front,
+// lay0, lay1. Stops when the first layer holding an anchor is found (its anchors then
 // replace L->anch), every wanted stair has a layer and every wanted monster lane is
 // reached, or nothing new is reached. Returns the anchor layer or -1.
 struct KB {
@@ -399,8 +421,8 @@ struct KB {
 // Lane l keeps rows l and (l < 6) 64 + l of the frontier, reach, known floor and anchors in
 // registers, as bfs() does (its layers by constant mod 3, rows 64.. only while the frontier is
 // near them). What the search looks for is one set of cells: a layer that meets none of them can
-// neither finish the search nor give a layer, so only the others run the checks. Reach, the layer
-// planes and the anchor rows are published at the end.
+// neither finish the search nor give a layer, so only the others run the checks. The reached cells
+// by layer mod 3 (0 in front, 1 in lay0, 2 in lay1) and the anchor rows are published at the end.
 __device__ __forceinline__ uint32_t row_word(Row r, int w) { return w == 0 ? r.a : w == 1 ? r.b : r.c; }
 __device__ __forceinline__ KB known_bfs(LCtx &c, bool want_anchor, int want_stairs, bool want_monster) {
     Ctx &x = c.x;
@@ -513,12 +535,12 @@ __device__ __forceinline__ KB known_bfs(LCtx &c, bool want_anchor, int want_stai
     };
     if (!check(0))
         while (!step(Const<1>{}) && !step(Const<2>{}) && !step(Const<0>{})) {}   // a layer adds a cell: at most N
-    row_st(sm->reach, lane, r0);
     row_st(sm->lay0, lane, e0);
     row_st(sm->lay1, lane, g0);
+    row_st(sm->front, lane, row_andn(r0, row_or(e0, g0)));   // layer % 3 == 0
     if (has1) {
-        row_st(sm->reach, 64 + lane, r1);
         row_st(sm->lay0, 64 + lane, e1); row_st(sm->lay1, 64 + lane, g1);
+        row_st(sm->front, 64 + lane, row_andn(r1, row_or(e1, g1)));
     }
     if (want_anchor) {   // the nearest layer's anchors; none reachable: the set is not needed
         row_st(L->anch, lane, r.alayer >= 0 ? a0 : zero);
@@ -530,20 +552,28 @@ __device__ __forceinline__ KB known_bfs(LCtx &c, bool want_anchor, int want_stai
 // route_first_step (learn.cu:248-264): back from target (at layer D) along the first
 // predecessor in direction order; the player's direction to the layer-1 cell. A reached
 // neighbour of a layer-D cell is at layer D-1 exactly when its layer mod 3 is (D-1) mod 3
-// (neighbours differ by at most one layer).
+// (neighbours differ by at most one layer), so a step back is one bit of one of the three
+// published class planes a neighbour (coordinates kept: no division per step).
 __device__ __forceinline__ int route_first_step(const LCtx &c, int target, int D) {
     const Ctx &x = c.x;
     const Smem *sm = x.sm;
     if (target < 0 || D < 0 || target == x.player) return -1;
-    int p = target;
+    int px = target % W, py = target / W;
+    const int dx = ddx(x.lane & 7), dy = ddy(x.lane & 7);
+    int m = (D - 1) % 3;   // D >= 1: the target is not the player
     for (; D > 1; D--) {
-        int q = nbr(p, x.lane & 7);
-        bool ok = x.lane < 8 && q >= 0 && bit(sm->reach, q) && lay3(sm, q) == (D - 1) % 3;
-        uint64_t mm = ballot(ok);
+        const uint32_t *plane = m == 0 ? sm->front : m == 1 ? sm->lay0 : sm->lay1;
+        const int qx = px + dx, qy = py + dy;
+        const bool in = inb(qx, qy) && x.lane < 8;
+        const uint64_t mm = ballot(in && bit_at(plane, qx, qy));
         if (!mm) return -1;
-        p = lane_val(q, __ffsll((unsigned long long)mm) - 1);
+        const int d = __ffsll((unsigned long long)mm) - 1;
+        px += ddx(d);
+        py += ddy(d);
+        m = m == 0 ? 2 : m - 1;
     }
-    uint64_t mm = ballot(x.lane < 8 && nbr(x.player, x.lane & 7) == p);
+    const int pl = x.player, sx = px - pl % W, sy = py - pl / W;   // the player's step to that cell
+    const uint64_t mm = ballot(x.lane < 8 && dx == sx && dy == sy);
     return mm ? __ffsll((unsigned long long)mm) - 1 : -1;
 }
 // First frontier-list entry in the nearest anchor layer (the reference's first
@@ -1011,7 +1041,7 @@ __global__ __launch_bounds__(64) void k_learn_init(uint8_t *state, int n, D1Conf
     observe_learn(c, obs ? obs + (size_t)env * D1L_OBS : nullptr, mask ? mask + (size_t)env * D1L_ACTIONS : nullptr);
 }
 template <int CLUMP>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_learn_step(uint8_t *state, int n, D1Config cfg, D1LTables t,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_learn_step(uint8_t *state, int n, D1Config cfg, D1LTables t,
                                                    const int64_t *actions, int limit, float *obs, float *mask,
                                                    float *out, const bool *active) {
     __shared__ LSmem L;
