@@ -830,14 +830,31 @@ __device__ __forceinline__ void observe_learn(LCtx &c, float *obs, float *mask) 
     const bool rest_ok = x.hp < cf->hp && cf->regen > 0 && !visible_awake(x);
     __syncthreads();
     float *ob = sm->stage;   // overlays the BFS bitmaps, which are no longer needed
-    for (int j = x.lane; j < D1L_OBS; j += 64) ob[j] = 0.f;
+    // the terrain and visibility planes from 15-column row patterns (viewed | floor << 15 in rq, view
+    // in cbase; cells outside the map are 0 in all of them); the fields between them start at zero
+    if (x.lane < 15) {
+        const int dy = x.lane - 7, y = py + dy, ay = iabs(dy);
+        uint32_t vf = 0, R = 0, Lf = 0;
+        if (y >= 0 && y < H)
+            vf = ((row_window17(row_ld(sm->viewed, y), px - 8) >> 1) & 0x7FFFu) |
+                 ((row_window17(row_ld(sm->floor, y), px - 8) >> 1) & 0x7FFFu) << 15;
+        if (dy >= 0) { R |= (uint32_t)(view_q(x, 0) >> (8 * ay)) & 0xFFu; Lf |= (uint32_t)(view_q(x, 1) >> (8 * ay)) & 0xFFu; }
+        if (dy <= 0) { R |= (uint32_t)(view_q(x, 3) >> (8 * ay)) & 0xFFu; Lf |= (uint32_t)(view_q(x, 2) >> (8 * ay)) & 0xFFu; }
+        sm->rq[x.lane] = vf;
+        c.L->cbase[x.lane] = (int)((__builtin_bitreverse32(Lf) >> 24) | (R << 7));
+    }
+    static_assert(O_ENEMY_HP == 225 && O_PROGRESS == O_VISIBLE + 225, "the planes' places");
+    for (int j = O_ENEMY_HP + x.lane; j < O_VISIBLE; j += 64) ob[j] = 0.f;
+    if (x.lane < D1L_OBS - O_PROGRESS) ob[O_PROGRESS + x.lane] = 0.f;
     __syncthreads();
-    for (int w = x.lane; w < 225; w += 64) {
-        int dx = w % 15 - 7, dy = w / 15 - 7, xx = px + dx, yy = py + dy;
-        if (!inb(xx, yy)) continue;
-        bool vw = bit_at(sm->viewed, xx, yy);
-        ob[w] = vw ? (bit_at(sm->floor, xx, yy) ? 1.f : -1.f) : 0.f;
-        ob[O_VISIBLE + w] = vis_rel(x, dx, dy) ? 1.f : 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const uint32_t w = 64u * k + (uint32_t)x.lane;
+        if (w >= 225u) continue;
+        const uint32_t r = (w * 4370u) >> 16, col = w - 15u * r;   // w / 15, exact below 256
+        const uint32_t t = sm->rq[r] >> col, v = (uint32_t)c.L->cbase[r] >> col;
+        ob[w] = t & 1u ? (t & 0x8000u ? 1.f : -1.f) : 0.f;
+        ob[O_VISIBLE + w] = v & 1u ? 1.f : 0.f;
     }
     if (lane_alive(c) && in_view(x, x.mpos)) {
         int dx = x.mpos % W - px, dy = x.mpos / W - py;
