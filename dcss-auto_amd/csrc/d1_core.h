@@ -114,6 +114,11 @@ __device__ __forceinline__ int nbr(int p, int d) {
     int x = p % W + ddx, y = p / W + ddy;
     return x >= 0 && x < W && y >= 0 && y < H ? y * W + x : -1;
 }
+// Direction d (N,E,S,W,NE,SE,SW,NW) as offsets: two bits of dx+1 / dy+1 per direction.
+constexpr uint32_t DXP = 1u | 2u << 2 | 1u << 4 | 0u << 6 | 2u << 8 | 2u << 10 | 0u << 12 | 0u << 14;
+constexpr uint32_t DYP = 0u | 1u << 2 | 2u << 4 | 1u << 6 | 0u << 8 | 2u << 10 | 2u << 12 | 0u << 14;
+__device__ __forceinline__ int ddx(int d) { return (int)((DXP >> (2 * d)) & 3u) - 1; }
+__device__ __forceinline__ int ddy(int d) { return (int)((DYP >> (2 * d)) & 3u) - 1; }
 __device__ __forceinline__ bool inb(int x, int y) { return x >= 0 && x < W && y >= 0 && y < H; }
 __device__ __forceinline__ bool bit_at(const uint32_t *bm, int x, int y) {
     return (bm[y * RW + (x >> 5)] >> (x & 31)) & 1u;
@@ -415,6 +420,7 @@ struct Ctx {
     // crowded step's monster phase holds enough live values that the registers spill.
     uint64_t visr[4];
     bool view_lds = false;
+    bool cfg_lds = false;   // *c is in LDS (a constant per kernel): fields may be read by a lane's index
     // this lane's monster (lane < count)
     int mpos, mhp, menergy, mawake, mkind;
     int mlay;    // absolute BFS layer of the monster's cell (FAR when not known)
@@ -630,6 +636,23 @@ __device__ __forceinline__ int kind_speed(const D1Config *c, int k) {
     s = k == 5 ? c->kinds[5].speed : s;
     return s;
 }
+__device__ __forceinline__ int lane_speed(const Ctx &x) {   // this lane's monster's, as kind_speed gives it
+    return x.cfg_lds ? x.c->kinds[(uint32_t)x.mkind < 6u ? x.mkind : 0].speed : kind_speed(x.c, x.mkind);
+}
+// The cell a directed action aims at and its bits, read together: tested one after the other
+// (view, occupancy, memory, floor, then floor again for the move) each waited out an LDS read.
+struct Aim {
+    int p;                      // -1: outside the map
+    bool floor, viewed, enemy;  // enemy: a living monster in view
+};
+__device__ __forceinline__ Aim aim_at(const Ctx &x, int dir) {
+    const int px = (int)((uint32_t)x.player % W), py = (int)((uint32_t)x.player / W);
+    const int dx = ddx(dir), dy = ddy(dir), nx = px + dx, ny = py + dy;
+    const bool in = inb(nx, ny);
+    const int w = in ? ny * RW + (nx >> 5) : 0;
+    const uint32_t f = x.sm->floor[w], v = x.sm->viewed[w], o = x.sm->occ[w], b = in ? 1u << (nx & 31) : 0u;
+    return {in ? ny * W + nx : -1, (f & b) != 0, (v & b) != 0, (o & b) != 0 && vis_rel(x, dx, dy)};
+}
 // gpu-d1/src/sim.h:130-163 (kind = the acting monster's kind)
 __device__ __forceinline__ void attack(Ctx &x, int kind) {
     const D1Config *c = x.c;
@@ -672,11 +695,6 @@ __device__ __forceinline__ bool walkable(const Ctx &x, int q) {
     return q >= 0 && bit(x.sm->floor, q) && q != x.player && !bit(x.sm->occ, q);
 }
 // ---------------------------------------------------------------- monster moves in coordinates
-// Direction d (N,E,S,W,NE,SE,SW,NW) as offsets: two bits of dx+1 / dy+1 per direction.
-constexpr uint32_t DXP = 1u | 2u << 2 | 1u << 4 | 0u << 6 | 2u << 8 | 2u << 10 | 0u << 12 | 0u << 14;
-constexpr uint32_t DYP = 0u | 1u << 2 | 2u << 4 | 1u << 6 | 0u << 8 | 2u << 10 | 2u << 12 | 0u << 14;
-__device__ __forceinline__ int ddx(int d) { return (int)((DXP >> (2 * d)) & 3u) - 1; }
-__device__ __forceinline__ int ddy(int d) { return (int)((DYP >> (2 * d)) & 3u) - 1; }
 // The bitmap words of one cell (x, y): walkable (floor, unoccupied, not the player), reached
 // by the distance field, its layer mod 3, queued by the repair search.
 struct Cell {

@@ -187,11 +187,12 @@ __device__ __forceinline__ void field_memo(Ctx &x) {
 
 // ---------------------------------------------------------------- one physical turn
 // gpu-d1/branches/d1-stairs-v2/src/learn.cu:684-827 with the v1 kill-all clear
-// (gpu-d1/src/learn.cu:549) as a switch. d: 0-7 move/bump, 8 wait, 18 descend.
+// (gpu-d1/src/learn.cu:549) as a switch. d: 0-7 move/bump (into the cell `to`), 8 wait, 18 descend.
 // Returns done; out8 = reward, done, clear, killed, hp, ticks, death, timeout.
 // `saw` (an awake monster was in view during the turn) is computed only when want_saw: REST
 // repeats read it, every other action ignores it.
-__device__ __forceinline__ bool primitive(Ctx &x, int d, float *out8, bool &saw, bool want_saw, const uint32_t *cells_g) {
+__device__ __forceinline__ bool primitive(Ctx &x, int d, const Aim &to, float *out8, bool &saw, bool want_saw,
+                                          const uint32_t *cells_g) {
     const D1Config *c = x.c;
     Smem *sm = x.sm;
     int milli = c->step_milli;
@@ -200,8 +201,8 @@ __device__ __forceinline__ bool primitive(Ctx &x, int d, float *out8, bool &saw,
     x.regen += c->regen;
     while (x.regen >= 100) { x.hp = imin(c->hp, x.hp + 1); x.regen -= 100; }
     if (d >= 0 && d < 8) {
-        int p = nbr(x.player, d);
-        if (p >= 0 && bit(sm->floor, p)) {
+        const int p = to.p;
+        if (to.floor) {
             uint64_t at = ballot(x.lane < c->count && x.mhp > 0 && x.mpos == p);
             if (at) {
                 int id = __ffsll((unsigned long long)at) - 1;
@@ -236,7 +237,7 @@ __device__ __forceinline__ bool primitive(Ctx &x, int d, float *out8, bool &saw,
             if (detects(x, pos) && x.lane == i) { x.mawake = 1; x.menergy = 70; }
         }
         if (mine && x.mhp > 0 && !x.mawake) x.menergy = -30000;
-        if (mine && x.mhp > 0) x.menergy += kind_speed(c, x.mkind);
+        if (mine && x.mhp > 0) x.menergy += lane_speed(x);
         x.menergy = (int16_t)x.menergy;
         uint64_t movers = ballot(mine && x.mhp > 0 && x.mawake && x.menergy >= 80 && cheb_u(x.mpos, x.player) > 1);
         if (movers) {
@@ -314,16 +315,16 @@ __device__ __forceinline__ void transition(Ctx &x, int action, float *out, const
     float total = 0.f, out8[8];
     for (int guard = 0; guard < 1 << 16; guard++) {
         int d = 8;
+        Aim to{-1, false, false, false};
         if (action >= 0 && action < 16) {
-            int dir = action % 8, p = nbr(x.player, dir);
-            bool enemy = p >= 0 && in_view(x, p) && bit(x.sm->occ, p);
-            bool valid = action < 8 ? p >= 0 && (!bit(x.sm->viewed, p) || bit(x.sm->floor, p)) && !enemy : enemy;
-            if (valid) d = dir; else invalid = true;
+            to = aim_at(x, action & 7);
+            const bool valid = action < 8 ? to.p >= 0 && (!to.viewed || to.floor) && !to.enemy : to.enemy;
+            if (valid) d = action & 7; else invalid = true;
         } else if (action == 17) invalid = x.hp >= c->hp || visible_awake(x) || c->regen <= 0;
         else if (action == 18) { if (stair_index(x) > 0) d = 18; else invalid = true; }
         else if (action != 16) invalid = true;
         bool saw = false;
-        bool done = primitive(x, d, out8, saw, action == 17, cells_g);
+        bool done = primitive(x, d, to, out8, saw, action == 17, cells_g);
         total += out8[0];
         if (done || invalid || action != 17) break;
         if (saw || x.hp >= c->hp) break;
@@ -672,6 +673,7 @@ __device__ __forceinline__ void step_worlds(Smem &sm, uint8_t *state, int n, int
     const int first = blk < g ? WPB * blk : WPB * g + (blk - g), last = imin(n, blk < g ? first + WPB : first + 1);
     Ctx x;
     x.sm = &sm; x.c = cfgp; x.rays = tab.ray_slots; x.nslots = tab.nslots; x.lane = lane_id();
+    x.cfg_lds = !CROWD;   // k_step's copy
     x.view_lds = CROWD;   // the crowded build keeps the player view in LDS
     x.stuck_cache = CROWD;   // and a complete distance field that depends on the player cell alone
     // Each world is loaded when the wave starts it. Fetching the next world's row while the

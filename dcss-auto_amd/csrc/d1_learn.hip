@@ -614,7 +614,7 @@ struct POut {
 };
 
 template <int CLUMP>
-__device__ __forceinline__ void primitive_learn(LCtx &c, int d, int limit, POut &o) {
+__device__ __forceinline__ void primitive_learn(LCtx &c, int d, const Aim &to, int limit, POut &o) {
     Ctx &x = c.x;
     Smem *sm = x.sm;
     const D1Config *cf = x.c;
@@ -624,8 +624,8 @@ __device__ __forceinline__ void primitive_learn(LCtx &c, int d, int limit, POut 
     x.regen += cf->regen;
     while (x.regen >= 100) { x.hp = imin(cf->hp, x.hp + 1); x.regen -= 100; }
     if (d >= 0 && d < 8) {
-        int p = nbr(x.player, d);
-        if (p >= 0 && bit(sm->floor, p)) {
+        const int p = to.p;
+        if (to.floor) {
             uint64_t at = ballot(lane_alive(c) && x.mpos == p);
             if (at) {
                 int id = __ffsll((unsigned long long)at) - 1;
@@ -741,15 +741,15 @@ __device__ __forceinline__ void transition_learn(LCtx &c, int action, int limit,
     POut o;
     for (int guard = 0; guard < (1 << 16); guard++) {
         int d = 8;
+        Aim to{-1, false, false, false};
         if (action >= 0 && action < 16) {
-            int dir = action % 8, p = nbr(x.player, dir);
-            bool enemy = p >= 0 && in_view(x, p) && bit(x.sm->occ, p);
-            bool valid = action < 8 ? p >= 0 && (!bit(x.sm->viewed, p) || bit(x.sm->floor, p)) && !enemy : enemy;
-            if (valid) d = dir; else invalid = 1;
+            to = aim_at(x, action & 7);
+            const bool valid = action < 8 ? to.p >= 0 && (!to.viewed || to.floor) && !to.enemy : to.enemy;
+            if (valid) d = action & 7; else invalid = 1;
         } else if (action == 17) invalid = x.hp >= cf->hp || visible_awake(x) || cf->regen <= 0;
         else if (action == 18) { if (stair_index(x) > 0) d = 18; else invalid = 1; }
         else if (action != 16) invalid = 1;
-        primitive_learn<CLUMP>(c, d, limit, o);
+        primitive_learn<CLUMP>(c, d, to, limit, o);
         elapsed++;
         total += o.reward;
         discounted += factor * o.reward;
