@@ -46,40 +46,59 @@ __global__ __launch_bounds__(256) void k_sample_dev(const float *__restrict__ lo
     sample_row(logits, i, k, ld, key0, key1, *t_dev + t_add, actions, logp);
 }
 
-// Reverse-time GAE. A workgroup owns 64 envs (a lane each); its eight waves take GC time steps
-// each, so that a round's GW * GC = 128 steps are all in flight at once. Each wave forms its
+// Reverse-time GAE. A workgroup owns 64 envs (a lane each); its up to eight waves take GC time
+// steps each, so that a round's 128 steps are all in flight at once. Each wave forms its
 // steps' deltas, then the waves run the recurrence in time order, the carry passing through
 // LDS: the only serial part is one product and one sum a step, in the order and rounding of
 // the reference's loop (bit-identical to it). One lane looping over T with a load level a step
 // left the kernel waiting on latency, 1,024 waves on the chip: 106.8 us at T = 128, n = 65,536
 // (143 MB) with the buffers out of cache, now 34.6 us (4.1 TB/s; a large copy reaches 5.1).
+// Short horizons get a kernel with only the waves they need, and a wave loads only the steps it
+// has. With eight waves always, the idle ones each loading step 0 sixteen times, T = 8 and 16
+// at 65,536 envs took 7.3 and 8.3 us (the one-lane loop: 3.6 and 5.9), now 3.2 and 4.1; at 64 to
+// 16,384 envs T = 8 took 3.2 to 3.6 us (the loop: 2.8 to 3.2), now 2.3 to 2.7; T = 128 is as before.
 constexpr int GW = 8, GC = 16;
-__global__ __launch_bounds__(64 * GW) void k_gae(const float *reward, const uint8_t *done, const float *value,
+template <int NW, int GC>   // waves a workgroup and time steps a wave; T > NW * GC only with the largest NW
+__global__ __launch_bounds__(64 * NW) void k_gae(const float *reward, const uint8_t *done, const float *value,
                                                  const float *bootstrap, int T, int n, float gamma, float gl, float *adv,
                                                  float *ret) {
-    __shared__ float first[GW][64], carry[64];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr bool MANY = NW > 1;
+    __shared__ float first[NW][64], carry[64];
+    const int lane = threadIdx.x & 63, wave = MANY ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     const int env = blockIdx.x * 64 + lane;
     const bool mine = env < n;
     const int i = mine ? env : n - 1;
     float after = bootstrap[i];   // value of the step after the round's last one
-    if (wave == 0) carry[lane] = 0.f;
-    for (int base = T - 1; base >= 0; base -= GW * GC) {
+    if (MANY && wave == 0) carry[lane] = 0.f;
+    for (int base = T - 1; base >= 0; base -= NW * GC) {
         const int t0 = base - GC * wave;   // this wave's steps t0, t0 - 1, .. ; wave 0 has the latest
-        const int cnt = min(GC, t0 + 1);
+        const int cnt = min(GC, t0 + 1);   // none: <= 0
         float r[GC], v[GC];
         uint32_t d[GC];
-#pragma unroll
-        for (int j = 0; j < GC; j++) {
-            const size_t o = (size_t)max(t0 - j, 0) * n + i;
+        auto load = [&](int j) {
+            const size_t o = (size_t)(t0 - j) * n + i;
             r[j] = reward[o];
             v[j] = value[o];
             d[j] = done[o];
+        };
+        if (cnt == GC) {
+#pragma unroll
+            for (int j = 0; j < GC; j++) load(j);
+        } else {
+#pragma unroll
+            for (int j = 0; j < GC; j++) {
+                r[j] = v[j] = 0.f;
+                d[j] = 0;
+                if (j < cnt) load(j);
+            }
         }
-        first[wave][lane] = v[GC - 1];   // read only where the wave's steps are all there
-        __syncthreads();
-        const float before = wave ? first[wave ? wave - 1 : 0][lane] : after;
-        after = first[GW - 1][lane];
+        float before = after;
+        if (MANY) {
+            first[wave][lane] = v[GC - 1];   // read only where the wave's steps are all there
+            __syncthreads();
+            if (wave) before = first[wave - 1][lane];
+            after = first[NW - 1][lane];     // of use only after a round whose waves are all full
+        }
         float c[GC];
 #pragma unroll
         for (int j = 0; j < GC; j++) {
@@ -90,9 +109,9 @@ __global__ __launch_bounds__(64 * GW) void k_gae(const float *reward, const uint
             r[j] = s - v[j];     // delta
             c[j] = gl * live;
         }
-        for (int w = 0; w < GW; w++) {
+        for (int w = 0; w < NW; w++) {
             if (w == wave && cnt > 0) {
-                float gae = carry[lane];
+                float gae = MANY ? carry[lane] : 0.f;
                 if (cnt == GC) {
 #pragma unroll
                     for (int j = 0; j < GC; j++) {
@@ -109,9 +128,9 @@ __global__ __launch_bounds__(64 * GW) void k_gae(const float *reward, const uint
                             r[j] = gae;
                         }
                 }
-                carry[lane] = gae;
+                if (MANY) carry[lane] = gae;
             }
-            __syncthreads();
+            if (MANY) __syncthreads();
         }
         if (mine) {
 #pragma unroll
@@ -263,8 +282,16 @@ int d1_gae(const float *reward, const uint8_t *done, const float *value, const f
            float gamma, float gamma_lambda, float *adv, float *returns, void *stream) {
     if (T < 0 || n < 0 || ((T && n) && (!reward || !done || !value || !bootstrap || !adv))) return D1_E_ARG;
     if (T == 0 || n == 0) return 0;
-    hipLaunchKernelGGL(d1p::k_gae, dim3((n + 63) / 64), dim3(64 * d1p::GW), 0, (hipStream_t)stream, reward, done, value,
-                       bootstrap, T, n, gamma, gamma_lambda, adv, returns);
+    auto go = [&](auto *kernel, int waves) {
+        hipLaunchKernelGGL(kernel, dim3((n + 63) / 64), dim3(64 * waves), 0, (hipStream_t)stream, reward, done, value,
+                           bootstrap, T, n, gamma, gamma_lambda, adv, returns);
+    };
+    using namespace d1p;   // the smallest kernel whose waves hold T steps
+    if (T <= 4) go(k_gae<1, 4>, 1);
+    else if (T <= GC) go(k_gae<1, GC>, 1);
+    else if (T <= 2 * GC) go(k_gae<2, GC>, 2);
+    else if (T <= 4 * GC) go(k_gae<4, GC>, 4);
+    else go(k_gae<GW, GC>, GW);
     return (int)hipGetLastError();
 }
 int d1_adv_norm(float *adv, int64_t count, const float *mean, const float *std, float eps, void *stream) {

@@ -1,4 +1,4 @@
-"""The GAE kernel at the edges of its split (64 envs a workgroup, eight waves of 16 time steps):
+"""The GAE kernel at the edges of its split (64 envs a workgroup, one to eight waves of 16 time steps):
 bit-equal to the fp32 loop, also where it writes over its inputs; and the normalisation of the
 advantages against its elementwise expression."""
 import importlib
@@ -9,7 +9,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(1, 1), (1, 33), (15, 64), (16, 65), (17, 63), (127, 100), (128, 64), (129, 1), (300, 130), (512, 7)]
+SHAPES = [(1, 1), (1, 33), (4, 65), (5, 64), (8, 129), (15, 64), (16, 65), (17, 63), (32, 64), (33, 65), (64, 64), (65, 63), (112, 3), (113, 70), (127, 100),
+          (128, 64), (129, 1), (144, 64), (145, 9), (300, 130), (512, 7)]
 
 
 def _draw(T, n):
