@@ -1,0 +1,39 @@
+"""FastPPO's host side, without a GPU: the kernels' wrappers are replaced by checks of what they would
+be given."""
+import importlib
+
+import pytest
+import torch
+
+ppo = importlib.import_module('dcss-auto_amd.ppo')
+
+
+@pytest.fixture
+def fast(monkeypatch):
+    """A FastPPO of 1,024-sample minibatches without its device buffers; GAE writes its step numbers and
+    fails where its output would run past the tensor that it is given."""
+    def gae(reward, done, value, bootstrap, gamma, lam, adv=None, returns=None):
+        for x in (adv, returns):
+            assert x.dtype == torch.float32 and x.is_contiguous() and x.numel() >= reward.numel()
+            x.view(-1)[:reward.numel()] = torch.arange(reward.numel(), dtype=torch.float32)
+        return adv, returns
+
+    monkeypatch.setattr(ppo.P, 'gae', gae)
+    monkeypatch.setattr(ppo.P, 'normalize_', lambda adv: adv.add_(0.5))
+    f = ppo.FastPPO.__new__(ppo.FastPPO)
+    f.gamma, f.lam, f.dev = 0.99, 0.95, torch.device('cpu')
+    return f
+
+
+def test_advantages_are_sized_by_the_rewards(fast):
+    """Rewards of more steps than T: the outputs hold all of them, and given ones that do not are refused."""
+    buf = ppo.RolloutBuffer(4, 6, device='cpu')
+    for name in ('rewards', 'values', 'dones'):
+        setattr(buf, name, torch.cat([getattr(buf, name)] * 2))
+    adv, ret = fast.advantages(buf)
+    assert torch.equal(ret, torch.arange(48.)) and torch.equal(adv, ret + 0.5)
+    full = torch.empty(48)
+    for bad in (torch.empty(24), torch.empty(96)[::2], torch.empty(48, dtype=torch.float64)):
+        for args in ((bad, full), (full, bad)):
+            with pytest.raises(ValueError):
+                fast.advantages(buf, *args)
