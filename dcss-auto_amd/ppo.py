@@ -246,8 +246,7 @@ class FastPPO:
         """The buffer's normalised advantages and its returns, flat (written to `adv` and `ret`
         when given: contiguous fp32 of the rewards' size)."""
         n = buf.rewards.numel()   # what the GAE kernel writes, whatever T and N say
-        if adv is None:
-            adv, ret = (torch.empty(n, dtype=torch.float32, device=buf.rewards.device) for _ in range(2))
+        adv, ret = (torch.empty(n, dtype=torch.float32, device=buf.rewards.device) if t is None else t for t in (adv, ret))
         for t in (adv, ret):
             if not (t.dtype == torch.float32 and t.is_contiguous() and t.numel() == n and t.device == buf.rewards.device):
                 raise ValueError('adv and ret must be contiguous fp32 of the size of the rewards, on their device')

@@ -37,3 +37,12 @@ def test_advantages_are_sized_by_the_rewards(fast):
         for args in ((bad, full), (full, bad)):
             with pytest.raises(ValueError):
                 fast.advantages(buf, *args)
+
+
+@pytest.mark.parametrize('given', [(), ('adv',), ('ret',), ('adv', 'ret')])
+def test_advantages_and_returns_are_each_made_when_not_given(fast, given):
+    buf = ppo.RolloutBuffer(4, 6, device='cpu')
+    out = {k: torch.empty(24) for k in given}
+    adv, ret = fast.advantages(buf, **out)
+    assert torch.equal(ret, torch.arange(24.)) and torch.equal(adv, ret + 0.5)
+    assert all(x is out[k] for k, x in (('adv', adv), ('ret', ret)) if k in given)
