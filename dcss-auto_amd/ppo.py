@@ -259,7 +259,12 @@ class FastPPO:
         if self.graph:
             if self._g is None or self._g_buf is not buf:
                 self._capture(buf)
-            adv, ret = self.advantages(buf, self._adv, self._ret)
+            if _is(self.advantages, _ADVANTAGES):
+                adv, ret = self.advantages(buf, self._adv, self._ret)
+            else:   # replaced by the program, as advantages(buf)
+                for mine, given in zip((self._adv, self._ret), self.advantages(buf)):
+                    mine.copy_(given)
+                adv, ret = self._adv, self._ret
             if not self._packed:   # weights replaced outside the step (a checkpoint load): the graph
                 self._struct(obs, actions, logp, adv, ret)   # only replays, so rebuild its weight copies here
         else:
@@ -279,3 +284,12 @@ class FastPPO:
         if self.nonfinite_steps():
             raise RuntimeError('Non-finite PPO loss')
         return terms
+
+
+def _is(method, function):
+    """Whether a bound method is `function` itself, not one that a subclass, an instance or a patched
+    class puts in its place."""
+    return getattr(method, '__func__', None) is function
+
+
+_ADVANTAGES = FastPPO.advantages

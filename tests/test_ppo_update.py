@@ -46,3 +46,50 @@ def test_advantages_and_returns_are_each_made_when_not_given(fast, given):
     adv, ret = fast.advantages(buf, **out)
     assert torch.equal(ret, torch.arange(24.)) and torch.equal(adv, ret + 0.5)
     assert all(x is out[k] for k, x in (('adv', adv), ('ret', ret)) if k in given)
+
+
+class _Graph:
+    replays = 0
+
+    def replay(self):
+        self.replays += 1
+
+
+def _ready(f, buf, graph):
+    """What update() finds after construction, and with graph=True after a capture."""
+    n = buf.T * buf.N
+    f.minibatch, f.epochs, f.graph, f.graph_steps = 1024, 3, graph, 16
+    f.perm, f._packed, f.head_out, f._args_key, f._g, f._g_buf = None, True, None, None, None, None
+    f.cursor, f.step_t, f.loss_parts = torch.zeros(2, dtype=torch.int32), torch.zeros(3), torch.zeros(128)
+    f.seen = []
+    f._struct = lambda *a: None
+    f._step = lambda obs, actions, logp, adv, ret: f.seen.append((adv.clone(), ret.clone(), f.perm.clone()))
+
+    def capture(b):
+        f._adv, f._ret = torch.zeros(n), torch.zeros(n)
+        f.perm = torch.zeros(n, dtype=torch.int64)
+        f._g, f._g_buf = _Graph(), b
+    f._capture = capture
+
+
+@pytest.mark.parametrize('graph', [False, True])
+@pytest.mark.parametrize('where', ['subclass', 'instance', 'class'])
+def test_update_calls_a_replaced_advantages_with_the_buffer_alone(fast, monkeypatch, graph, where):
+    buf = ppo.RolloutBuffer(4, 512, device='cpu')
+    mine = torch.randn(2048), torch.randn(2048)
+
+    def advantages(self, b):
+        assert b is buf
+        return mine
+    _ready(fast, buf, graph)
+    if where == 'subclass':
+        fast.__class__ = type('Own', (ppo.FastPPO,), dict(advantages=advantages))
+    elif where == 'instance':
+        fast.advantages = lambda b: advantages(fast, b)
+    else:
+        monkeypatch.setattr(ppo.FastPPO, 'advantages', advantages)
+    fast.update(buf, generator=torch.Generator().manual_seed(1))
+    if graph:
+        assert fast._g.replays == 3 and torch.equal(fast._adv, mine[0]) and torch.equal(fast._ret, mine[1])
+    else:
+        assert len(fast.seen) == 6 and all(torch.equal(a, mine[0]) and torch.equal(r, mine[1]) for a, r, _ in fast.seen)
