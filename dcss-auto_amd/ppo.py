@@ -271,9 +271,12 @@ class FastPPO:
             adv, ret = self.advantages(buf)
         steps = n // self.minibatch            # a ragged tail is dropped (T*N is a multiple in C4)
         for _ in range(self.epochs):
-            if self.perm is None or self.perm.numel() != n:
-                self.perm = torch.empty(n, dtype=torch.int64, device=self.dev)
-            self.set_order(torch.randperm(n, out=self.perm, generator=generator))
+            if _is(self.set_order, _SET_ORDER):   # straight into the order buffer
+                if self.perm is None or self.perm.numel() != n:
+                    self.perm = torch.empty(n, dtype=torch.int64, device=self.dev)
+                self.set_order(torch.randperm(n, out=self.perm, generator=generator))
+            else:   # replaced by the program: an order of its own, which it may keep
+                self.set_order(torch.randperm(n, device=self.dev, generator=generator))
             if self.graph:
                 for _ in range(steps // self._graph_len(n)):
                     self._g.replay()
@@ -292,4 +295,4 @@ def _is(method, function):
     return getattr(method, '__func__', None) is function
 
 
-_ADVANTAGES = FastPPO.advantages
+_ADVANTAGES, _SET_ORDER = FastPPO.advantages, FastPPO.set_order

@@ -93,3 +93,20 @@ def test_update_calls_a_replaced_advantages_with_the_buffer_alone(fast, monkeypa
         assert fast._g.replays == 3 and torch.equal(fast._adv, mine[0]) and torch.equal(fast._ret, mine[1])
     else:
         assert len(fast.seen) == 6 and all(torch.equal(a, mine[0]) and torch.equal(r, mine[1]) for a, r, _ in fast.seen)
+
+
+@pytest.mark.parametrize('graph', [False, True])
+def test_a_replaced_set_order_may_keep_the_orders_it_is_given(fast, graph):
+    """The same orders as randperm draws from the generator, each in a tensor of its own."""
+    buf = ppo.RolloutBuffer(4, 512, device='cpu')
+    _ready(fast, buf, graph)
+    kept, orig = [], fast.set_order
+
+    def set_order(perm):
+        kept.append(perm)
+        orig(perm)
+    fast.set_order = set_order
+    fast.update(buf, generator=torch.Generator().manual_seed(5))
+    g = torch.Generator().manual_seed(5)
+    assert len(kept) == 3 and all(torch.equal(k, torch.randperm(2048, generator=g)) for k in kept)
+    assert torch.equal(fast.perm, kept[-1])
