@@ -151,13 +151,17 @@ class FastPPO:
         self.perm = None
         self.head_out = None   # [minibatch, 17] fp32: when set, each step writes its head outputs here
         self._packed = False
-        self._g = self._g_buf = None
+        self._g = self._g_buf = self._g_key = None
         self._args = self._args_key = None
+
+    def _key(self, obs, actions, logp, adv, ret):
+        """What a step's launches hold: the addresses they read and write, and the sample count."""
+        return (obs.data_ptr(), actions.data_ptr(), logp.data_ptr(), adv.data_ptr(), ret.data_ptr(),
+                self.perm.data_ptr(), obs.shape[0], 0 if self.head_out is None else self.head_out.data_ptr())
 
     def _struct(self, obs, actions, logp, adv, ret):
         from . import _lib
-        key = (obs.data_ptr(), actions.data_ptr(), logp.data_ptr(), adv.data_ptr(), ret.data_ptr(),
-               self.perm.data_ptr(), obs.shape[0], 0 if self.head_out is None else self.head_out.data_ptr())
+        key = self._key(obs, actions, logp, adv, ret)
         if self._args_key != key:
             F = self.flat
             if obs.shape[1] != OBS or not obs.is_contiguous() or obs.dtype != torch.uint8:
@@ -231,7 +235,7 @@ class FastPPO:
             raise ValueError('the buffer holds fewer samples than one minibatch')
         self._adv = torch.zeros(n, device=self.dev)
         self._ret = torch.zeros(n, device=self.dev)
-        if self.perm is None or self.perm.numel() != n:
+        if self.perm is None or self.perm.shape != (n,):
             self.perm = torch.zeros(n, dtype=torch.int64, device=self.dev)
         obs, actions, logp = self._views(buf)
         args = self._struct(obs, actions, logp, self._adv, self._ret)
@@ -241,6 +245,7 @@ class FastPPO:
             for _ in range(self._graph_len(n)):
                 self._step(obs, actions, logp, self._adv, self._ret)
         self._g, self._g_buf, self._g_args = g, buf, args
+        self._g_key = self._key(obs, actions, logp, self._adv, self._ret)
 
     def advantages(self, buf, adv=None, ret=None):
         """The buffer's normalised advantages and its returns, flat (written to `adv` and `ret`
@@ -256,8 +261,13 @@ class FastPPO:
     def update(self, buf, generator=None):
         n = buf.T * buf.N
         obs, actions, logp = self._views(buf)
+        if self.perm is None or self.perm.shape != (n,):
+            self.perm = torch.empty(n, dtype=torch.int64, device=self.dev)
         if self.graph:
-            if self._g is None or self._g_buf is not buf:
+            # the graph holds addresses: another order buffer (set_order with another size) or a
+            # tensor of the buffer that was replaced needs a new one
+            if self._g is None or self._g_buf is not buf or \
+                    self._g_key != self._key(obs, actions, logp, self._adv, self._ret):
                 self._capture(buf)
             if _is(self.advantages, _ADVANTAGES):
                 adv, ret = self.advantages(buf, self._adv, self._ret)
@@ -272,8 +282,6 @@ class FastPPO:
         steps = n // self.minibatch            # a ragged tail is dropped (T*N is a multiple in C4)
         for _ in range(self.epochs):
             if _is(self.set_order, _SET_ORDER):   # straight into the order buffer
-                if self.perm is None or self.perm.numel() != n:
-                    self.perm = torch.empty(n, dtype=torch.int64, device=self.dev)
                 self.set_order(torch.randperm(n, out=self.perm, generator=generator))
             else:   # replaced by the program: an order of its own, which it may keep
                 self.set_order(torch.randperm(n, device=self.dev, generator=generator))

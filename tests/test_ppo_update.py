@@ -67,8 +67,11 @@ def _ready(f, buf, graph):
 
     def capture(b):
         f._adv, f._ret = torch.zeros(n), torch.zeros(n)
-        f.perm = torch.zeros(n, dtype=torch.int64)
+        if f.perm is None or f.perm.shape != (n,):
+            f.perm = torch.zeros(n, dtype=torch.int64)
         f._g, f._g_buf = _Graph(), b
+        f._g.reads = [x.data_ptr() for x in (f.perm, b.obs, b.actions, b.logp)]
+        f._g_key = f._key(*f._views(b), f._adv, f._ret)
     f._capture = capture
 
 
@@ -110,3 +113,25 @@ def test_a_replaced_set_order_may_keep_the_orders_it_is_given(fast, graph):
     g = torch.Generator().manual_seed(5)
     assert len(kept) == 3 and all(torch.equal(k, torch.randperm(2048, generator=g)) for k in kept)
     assert torch.equal(fast.perm, kept[-1])
+
+
+def test_update_captures_again_when_the_graph_holds_other_buffers(fast):
+    """An order of another size between two updates, and a replaced tensor of the buffer: the captured
+    launches would read the old allocations."""
+    buf = ppo.RolloutBuffer(4, 512, device='cpu')
+    _ready(fast, buf, True)
+
+    def update():
+        fast.update(buf, generator=torch.Generator().manual_seed(1))
+        assert fast._g.reads == [x.data_ptr() for x in (fast.perm, buf.obs, buf.actions, buf.logp)]
+        return fast._g
+    first, old_perm = update(), fast.perm
+    assert update() is first                      # nothing changed: the same graph
+    fast.set_order(torch.arange(1024))
+    second = update()
+    assert second is not first and fast.perm is not old_perm and fast.perm.shape == (2048,)
+    old_logp, buf.logp = buf.logp, buf.logp.clone()
+    assert update() is not second and old_logp is not buf.logp
+    fast.set_order(torch.arange(2048).view(2, 1024))   # as many values in another shape
+    update()
+    assert fast.perm.shape == (2048,)
