@@ -35,6 +35,7 @@ from .env import Env
 # stuck-cache radii to that memo (rows of 40 monsters 5,632 -> 5,696 bytes); version-1 files
 # carry no 'format' key.
 CHECKPOINT_FORMAT = 3
+_ENV_STEP = Env.step
 
 
 class Trainer:
@@ -82,7 +83,7 @@ class Trainer:
         b1, b2, b3 = self.bias
         # the step writes the reward and done rows itself (two copy launches a step), unless the
         # environment has a step() of its own
-        plain = type(env) is Env and 'step' not in vars(env)
+        plain = type(env) is Env and ppo_mod._is(env.step, _ENV_STEP)
         buf.obs[0].copy_(self.next_obs)
         for k in range(self.T):   # forward + sample in one kernel, the counter step read on the device
             P.policy_fwd_sample(buf.obs[k], self.wpk, b1, b2, b3, self.seed, k, buf.actions[k], buf.logp[k],

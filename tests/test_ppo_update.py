@@ -1,5 +1,5 @@
-"""FastPPO's host side, without a GPU: the kernels' wrappers are replaced by checks of what they would
-be given."""
+"""The host side of FastPPO's update and of the trainer's rollout, without a GPU: the kernels' wrappers are
+replaced by checks of what they would be given."""
 import importlib
 
 import pytest
@@ -135,3 +135,26 @@ def test_update_captures_again_when_the_graph_holds_other_buffers(fast):
     fast.set_order(torch.arange(2048).view(2, 1024))   # as many values in another shape
     update()
     assert fast.perm.shape == (2048,)
+
+
+@pytest.mark.parametrize('where', ['instance', 'class', None])
+def test_rollout_steps_through_a_replaced_step(pkg, monkeypatch, where):
+    """Env.step wrapped on the instance or on the class (to count or log steps) sees every step; the
+    class as it is goes through step_into."""
+    train = importlib.import_module('dcss-auto_amd.train')
+    monkeypatch.setattr(train.P, 'policy_fwd_sample', lambda *a, **k: None)
+    monkeypatch.setattr(train.P, 'policy_fwd', lambda *a, **k: None)
+    calls = []
+    env = pkg.Env.__new__(pkg.Env)
+    env.out = torch.zeros(6, 8)
+    monkeypatch.setattr(pkg.Env, 'step_into', lambda self, *a: calls.append('step_into'))
+    if where == 'instance':
+        env.step = lambda actions, obs: calls.append('step')
+    elif where == 'class':
+        monkeypatch.setattr(pkg.Env, 'step', lambda self, actions, obs: calls.append('step'))
+    t = train.Trainer.__new__(train.Trainer)
+    t.buf, t.env, t.T, t.seed = ppo.RolloutBuffer(4, 6, device='cpu'), env, 4, 1
+    t.bias, t.wpk, t.logits = (None, None, None), None, None
+    t.t_dev, t.next_obs = torch.zeros(1, dtype=torch.int32), torch.zeros(6, 1800, dtype=torch.uint8)
+    t._rollout_body()
+    assert calls == ['step' if where else 'step_into'] * 4
