@@ -105,6 +105,21 @@ def test_parity_multimap_clumped(L, O):
     assert ref.scalar('placement_clumped').any()
 
 
+@pytest.mark.parametrize('clump', [0, 1])
+def test_parity_at_the_maps_edges(L, O, clump):
+    """Windows cut off by every edge of the map: a floor without walls, strips of nine columns along the left
+    and right edges and of nine rows along the top and bottom. In the strips' worlds every player
+    stands in columns 0-8 or 71-79, or in rows 0-8 or 61-69, all the time."""
+    open_floor, columns, rows = (np.zeros((70, 80), np.uint8) for _ in range(3))
+    open_floor[:] = 1
+    columns[:, :9] = columns[:, 71:] = 1
+    rows[:9] = rows[61:] = 1
+    env, ref = run_parity(L, O, [m.reshape(-1) for m in (columns, open_floor, rows)], batch=60, steps=150, seed=23,
+                          clump=clump, map_filter=-2, check_state_every=2)
+    assert len(set(ref.scalar('map_id').tolist())) == 3
+    assert ref.scalar('episode').sum() > 0 and (ref.scalar('floor_seen') > 200).any()
+
+
 def test_parity_rests_into_the_deadline(L, O):
     """60-turn episodes with a REST decision every other step: many-turn rests end at full
     HP or run into the deadline (the turn that reaches it ends the episode and resets the
