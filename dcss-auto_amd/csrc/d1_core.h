@@ -51,7 +51,6 @@ __device__ __forceinline__ int lane_id() { return (int)threadIdx.x; }
 __device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
 __device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
 __device__ __forceinline__ int iabs(int a) { return a < 0 ? -a : a; }
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ int lane_val(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
 __device__ __forceinline__ uint64_t ballot(bool b) { return __ballot(b); }
 // DPP lane moves (GFX9 data-parallel primitives, no LDS round trip). `id` fills the lanes
@@ -683,16 +682,11 @@ __device__ __forceinline__ void attack(Ctx &x, int kind) {
     damage = imax(0, damage - saved);
     x.hp -= damage;
 }
-// BFS layer mod 3 of cell q (meaningful where reach is set)
-__device__ __forceinline__ int lay3(const Smem *sm, int q) { return (int)bit(sm->lay0, q) | ((int)bit(sm->lay1, q) << 1); }
 // layer(q) - layer(r) from the layers mod 3 of two reached cells whose layers differ by at
 // most one (8-neighbours on the BFS graph): -1, 0 or +1
 __device__ __forceinline__ int step3(int mq, int mr) {
     const int d = mq - mr;
     return d == 1 || d == -2 ? 1 : (d == -1 || d == 2 ? -1 : 0);
-}
-__device__ __forceinline__ bool walkable(const Ctx &x, int q) {
-    return q >= 0 && bit(x.sm->floor, q) && q != x.player && !bit(x.sm->occ, q);
 }
 // ---------------------------------------------------------------- monster moves in coordinates
 // The bitmap words of one cell (x, y): walkable (floor, unoccupied, not the player), reached

@@ -83,7 +83,6 @@ __device__ __forceinline__ Row row_xor(Row x, Row y) { return {x.a ^ y.a, x.b ^ 
 __device__ __forceinline__ int lanes_below(uint64_t m, int lane) {
     return __popcll(m & ((1ULL << lane) - 1ULL));
 }
-__device__ __forceinline__ bool floor_b(const LCtx &c, int p) { return p >= 0 && bit(c.x.sm->floor, p); }
 
 // ---------------------------------------------------------------- view from the LOS table
 // in_view (learn.cu:192-198): bit (dy+8)*17+dx+8 of the player's LOS row; lane j
@@ -134,12 +133,6 @@ __device__ __forceinline__ void anchors_all(LCtx &c) {
     for (int y = c.x.lane; y < H; y += 64) row_st(c.L->anch, y, anchor_row(c.x.sm, y));
     __syncthreads();
 }
-__device__ __forceinline__ int popc_below(Row r, int xx) {
-    if (xx < 32) return __popc(r.a & ((1u << xx) - 1u));
-    if (xx < 64) return __popc(r.a) + __popc(r.b & ((1u << (xx - 32)) - 1u));
-    return __popc(r.a) + __popc(r.b) + __popc(r.c & ((1u << (xx - 64)) - 1u));
-}
-
 // columns x0 .. x0 + 16 of an 80-bit row (x0 from -8); columns outside the map read 0
 __device__ __forceinline__ uint32_t row_window17(Row r, int x0) {
     if (x0 < 0) return (r.a << -x0) & 0x1FFFFu;
@@ -587,7 +580,6 @@ __device__ __forceinline__ int first_hit(const LCtx &c) {
     }
     return -1;
 }
-__device__ __forceinline__ int known_stairs_l(const Ctx &x) { return known_stairs(x); }
 // seen-stair mask (bit k)
 __device__ __forceinline__ int seen_stairs(const Ctx &x) {
     int m = 0;
