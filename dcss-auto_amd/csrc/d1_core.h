@@ -221,25 +221,9 @@ __device__ __forceinline__ uint32_t pcg_out(uint64_t old) {
 __device__ __noinline__ uint32_t pcg_lane(uint64_t st, uint64_t inc, int lane) {
     return pcg_out(kJump.a[lane] * st + kJump.c[lane] * inc);
 }
-// Word idx%4 of Philox4x32-10(ctr = {idx/4, t, env, dom}, key = {key0, key1})
+// Block `blk` of Philox4x32-10(ctr = {blk, t, env, dom}, key = {key0, key1}): four words
 // (Salmon et al., SC'11: multipliers 0xD2511F53/0xCD9E8D57, Weyl increments
 // 0x9E3779B9/0xBB67AE85).
-__device__ __noinline__ uint32_t philox_lane(uint32_t key0, uint32_t key1, uint32_t t, uint32_t env, uint32_t dom,
-                                             uint32_t idx) {
-    uint32_t c0 = idx >> 2, c1 = t, c2 = env, c3 = dom, k0 = key0, k1 = key1;
-#pragma unroll
-    for (int r = 0; r < 10; r++) {
-        uint32_t hi0 = __umulhi(0xD2511F53u, c0), lo0 = 0xD2511F53u * c0;
-        uint32_t hi1 = __umulhi(0xCD9E8D57u, c2), lo1 = 0xCD9E8D57u * c2;
-        uint32_t n0 = hi1 ^ c1 ^ k0, n2 = hi0 ^ c3 ^ k1;
-        c0 = n0; c1 = lo1; c2 = n2; c3 = lo0;
-        k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
-    }
-    uint32_t j = idx & 3u;
-    return j == 0 ? c0 : j == 1 ? c1 : j == 2 ? c2 : c3;
-}
-
-// all four words of block `blk` of the stream
 __device__ __forceinline__ void philox_block(uint32_t key0, uint32_t key1, uint32_t t, uint32_t env, uint32_t dom,
                                              uint32_t blk, uint32_t (&w)[4]) {
     uint32_t c0 = blk, c1 = t, c2 = env, c3 = dom, k0 = key0, k1 = key1;
@@ -252,6 +236,14 @@ __device__ __forceinline__ void philox_block(uint32_t key0, uint32_t key1, uint3
         k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
     }
     w[0] = c0; w[1] = c1; w[2] = c2; w[3] = c3;
+}
+// Word idx of the stream: word idx%4 of block idx/4.
+__device__ __noinline__ uint32_t philox_lane(uint32_t key0, uint32_t key1, uint32_t t, uint32_t env, uint32_t dom,
+                                             uint32_t idx) {
+    uint32_t w[4];
+    philox_block(key0, key1, t, env, dom, idx >> 2, w);
+    const uint32_t j = idx & 3u;
+    return j == 0 ? w[0] : j == 1 ? w[1] : j == 2 ? w[2] : w[3];
 }
 
 struct Rng {
