@@ -600,18 +600,21 @@ __global__ __launch_bounds__(256) void k_policy(const uint8_t *__restrict__ obs,
 // waves split the hidden units: wave w computes units 32w..32w+31 of every layer for all of
 // them. A wave then reads only its own row block's weight fragments, which go from L2 straight
 // to registers (a ring, three or five chunks ahead), while the observations, which every wave
-// needs, are widened once into fragment-ordered LDS. What bounds it is the stream of all of W1
-// (928 KB, 6 us at a CU's 64 B/clk) into each CU and the serial chain of loads, layers and the
-// draw, not MFMA work or the ring's depth. k_policy -> here, forward + sample: 46.5 -> 14.1 us
-// at 1,024 rows, 46.9 -> 18.1 at 8,192 (TB = 1), 47.1 -> 26.1 at 16,384 (TB = 2); with the
-// autoregressive head 57.4 -> 19.1, 58.1 -> 23.7 and 60.4 -> 33.8.
+// needs, are widened once into fragment-ordered LDS. What bounds it is the chain of one
+// workgroup: all of W1 into its CU (928 KB, 6 us at the 64 B/clk of a CU's L1; counted, 1.16 MB of
+// L1 misses a workgroup, no LDS bank conflict), the layers one after the other, the draw. MFMA is busy
+// 3.5 us of it. k_policy -> here, forward + sample, launches of one graph: 47.2 -> 14.0 us at 1,024
+// rows, 47.4 -> 16.0 at 8,192 (TB = 1), 48.5 -> 25.3 at 16,384 (TB = 2); with the autoregressive head
+// 60.5 -> 20.5, 60.7 -> 23.3 and 64.4 -> 32.2.
 //   x      the rows' bytes are all loaded at the start (16 bytes a lane and piece) and stored
 //          as widened fragments, 64 KB of chunks a phase into two buffers; TB = 1 fits both
 //          of its phases, TB = 2 stores phase p + 2 where phase p was.
 //   h1, h2 leave a wave as the two B fragments (K steps 2w, 2w + 1) that to_frags of k_policy
 //          builds, through LDS; the same packed weights, K order and accumulation order give
 //          bit-identical outputs.
-//   head   wave 0 alone (both sample blocks at TB = 2), with k_policy's epilogues.
+//   head   wave w < TB takes sample block w, with k_policy's epilogues (both blocks on wave 0 left the
+//          CU's other waves waiting for its tanh and draws: 35.8 us for the autoregressive head at
+//          16,384 rows, 32.2 with a wave a block).
 template <int MODE, int TB>
 __global__ __launch_bounds__(512) void k_policy_small(const uint8_t *__restrict__ obs, int M,
                                                       const uint16_t *__restrict__ wpk, const uint16_t *__restrict__ b1,
@@ -766,19 +769,17 @@ __global__ __launch_bounds__(512) void k_policy_small(const uint8_t *__restrict_
         for (int a = 0; a < TB; a++) acc[a] = mfma(as_bf(w2f[s]), as_bf(xs[(a * 16 + s) * 64 + lane]), acc[a]);
     to_lds(bl + 256, xs + O_H2);
     __syncthreads();
-    if (wave) return;
+    if (wave >= TB) return;
 
-    bf16x8 hf[TB][16];
+    bf16x8 hf[1][16];
 #pragma unroll
-    for (int a = 0; a < TB; a++)
-#pragma unroll
-        for (int s = 0; s < 16; s++) hf[a][s] = as_bf(xs[O_H2 + (a * 16 + s) * 64 + lane]);
-    const int me = min(M, m0 + 32 * TB);
+    for (int s = 0; s < 16; s++) hf[0][s] = as_bf(xs[O_H2 + (wave * 16 + s) * 64 + lane]);
+    const int mw = m0 + 32 * wave, me = min(M, mw + 32);   // wave w: the head and the draw of sample block w
     if constexpr (AR)
-        ar_epilogue<TB>(xs + O_HEAD, xs + O_AR, bl, hf, lane, lr, lh, m0, me, key0, key1, tstep, value, actions, logp, ar);
+        ar_epilogue<1>(xs + O_HEAD, xs + O_AR, bl, hf, lane, lr, lh, mw, me, key0, key1, tstep, value, actions, logp, ar);
     else
-        head_epilogue<SAMPLE, TB>(xs + O_HEAD, bl, hf, lane, lr, lh, m0, me, key0, key1, tstep, logits, value, actions,
-                                  logp);
+        head_epilogue<SAMPLE, 1>(xs + O_HEAD, bl, hf, lane, lr, lh, mw, me, key0, key1, tstep, logits, value, actions,
+                                 logp);
 }
 
 // Packed weights, one thread per element (gather form: every element is written, padding
@@ -830,7 +831,12 @@ __global__ __launch_bounds__(256) void k_policy_pack_ar(const uint16_t *__restri
 // the 256 CUs at once (LDS allows each one a CU): 256 x 32 rows, then 256 x 64; past them the
 // next kernel wins at once (8,224 rows: 29.6 us with TB = 1, 21.4 with TB = 2; 16,416: 45.8
 // with TB = 2, 47.1 on k_policy, which from there on also keeps the fewest CU-microseconds a
-// row: callers run two such batches side by side).
+// row). Two batches side by side on two streams, a pair on k_policy -> here: 49.8 -> 28.6 us at
+// 2 x 8,192 rows, 49.8 -> 38.4 at 2 x 12,288, 49.9 -> 48.9 at 2 x 16,384 (autoregressive 65.5 ->
+// 42.3, 48.8 and 62.5); step and forward of two row ranges as two chains 100.0 -> 61.3 us at
+// 2 x 8,192 worlds and 112.5 -> 91.8 at 2 x 16,384 (the step's own gains included). The line is for
+// one or two batches at a time: three or four large ones fit the chip together on k_policy, and take
+// longer here (4 x 8,192 rows 52.8 -> 58.8 us, 4 x 16,384 61.3 -> 98.6; 4 x 4,096 52.2 -> 31.0).
 constexpr int SMALL1 = 8192, SMALL2 = 16384;
 template <int MODE>
 static int launch_policy(const uint8_t *obs, int M, const void *wpk, const void *b1, const void *b2, const void *b3,
