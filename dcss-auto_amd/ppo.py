@@ -151,7 +151,7 @@ class FastPPO:
         self.perm = None
         self.head_out = None   # [minibatch, 17] fp32: when set, each step writes its head outputs here
         self._packed = False
-        self._g = self._g_buf = self._g_key = None
+        self._g = self._g_buf = self._g_key = self._adv = self._ret = None
         self._args = self._args_key = None
 
     def _key(self, obs, actions, logp, adv, ret):
@@ -233,8 +233,9 @@ class FastPPO:
         n = buf.T * buf.N
         if n < self.minibatch:
             raise ValueError('the buffer holds fewer samples than one minibatch')
-        self._adv = torch.zeros(n, device=self.dev)
-        self._ret = torch.zeros(n, device=self.dev)
+        if self._adv is None or self._adv.numel() != n:
+            self._adv = torch.zeros(n, device=self.dev)
+            self._ret = torch.zeros(n, device=self.dev)
         if self.perm is None or self.perm.shape != (n,):
             self.perm = torch.zeros(n, dtype=torch.int64, device=self.dev)
         obs, actions, logp = self._views(buf)
@@ -250,35 +251,41 @@ class FastPPO:
     def advantages(self, buf, adv=None, ret=None):
         """The buffer's normalised advantages and its returns, flat (written to `adv` and `ret`
         when given: contiguous fp32 of the rewards' size)."""
-        n = buf.rewards.numel()   # what the GAE kernel writes, whatever T and N say
-        adv, ret = (torch.empty(n, dtype=torch.float32, device=buf.rewards.device) if t is None else t for t in (adv, ret))
+        n, device = buf.rewards.numel(), buf.rewards.device   # what the GAE kernel writes, whatever T and N say
+        adv, ret = (torch.empty(n, dtype=torch.float32, device=device) if t is None else t for t in (adv, ret))
         for t in (adv, ret):
-            if not (t.dtype == torch.float32 and t.is_contiguous() and t.numel() == n and t.device == buf.rewards.device):
+            if not (t.dtype == torch.float32 and t.is_contiguous() and t.numel() == n and t.device == device):
                 raise ValueError('adv and ret must be contiguous fp32 of the size of the rewards, on their device')
+        return self._advantages(buf, adv, ret)
+
+    def _advantages(self, buf, adv, ret):
         P.gae(buf.rewards, buf.dones, buf.values, buf.bootstrap, self.gamma, self.lam, adv=adv, returns=ret)
         return P.normalize_(adv), ret
 
     def update(self, buf, generator=None):
         n = buf.T * buf.N
         obs, actions, logp = self._views(buf)
-        if self.perm is None or self.perm.shape != (n,):
-            self.perm = torch.empty(n, dtype=torch.int64, device=self.dev)
         if self.graph:
-            # the graph holds addresses: another order buffer (set_order with another size) or a
-            # tensor of the buffer that was replaced needs a new one
-            if self._g is None or self._g_buf is not buf or \
-                    self._g_key != self._key(obs, actions, logp, self._adv, self._ret):
+            if self._g is None or self._g_buf is not buf:
                 self._capture(buf)
             if _is(self.advantages, _ADVANTAGES):
-                adv, ret = self.advantages(buf, self._adv, self._ret)
+                if buf.rewards.numel() != n or buf.rewards.device != self._adv.device:
+                    raise ValueError('the buffer holds another number of rewards than T x N, or on another device')
+                adv, ret = self._advantages(buf, self._adv, self._ret)
             else:   # replaced by the program, as advantages(buf)
                 for mine, given in zip((self._adv, self._ret), self.advantages(buf)):
                     mine.copy_(given)
                 adv, ret = self._adv, self._ret
+            # the graph holds addresses: another order buffer (set_order with another size) or a
+            # tensor of the buffer that was replaced needs a new one (looked at once GAE is queued)
+            if self.perm.shape != (n,) or self._g_key != self._key(obs, actions, logp, adv, ret):
+                self._capture(buf)
             if not self._packed:   # weights replaced outside the step (a checkpoint load): the graph
                 self._struct(obs, actions, logp, adv, ret)   # only replays, so rebuild its weight copies here
         else:
             adv, ret = self.advantages(buf)
+            if self.perm is None or self.perm.shape != (n,):
+                self.perm = torch.empty(n, dtype=torch.int64, device=self.dev)
         steps = n // self.minibatch            # a ragged tail is dropped (T*N is a multiple in C4)
         for _ in range(self.epochs):
             if _is(self.set_order, _SET_ORDER):   # straight into the order buffer

@@ -59,14 +59,15 @@ def _ready(f, buf, graph):
     """What update() finds after construction, and with graph=True after a capture."""
     n = buf.T * buf.N
     f.minibatch, f.epochs, f.graph, f.graph_steps = 1024, 3, graph, 16
-    f.perm, f._packed, f.head_out, f._args_key, f._g, f._g_buf = None, True, None, None, None, None
+    f.perm, f._packed, f.head_out, f._args_key, f._g, f._g_buf, f._adv = None, True, None, None, None, None, None
     f.cursor, f.step_t, f.loss_parts = torch.zeros(2, dtype=torch.int32), torch.zeros(3), torch.zeros(128)
     f.seen = []
     f._struct = lambda *a: None
     f._step = lambda obs, actions, logp, adv, ret: f.seen.append((adv.clone(), ret.clone(), f.perm.clone()))
 
     def capture(b):
-        f._adv, f._ret = torch.zeros(n), torch.zeros(n)
+        if f._adv is None or f._adv.numel() != n:
+            f._adv, f._ret = torch.zeros(n), torch.zeros(n)
         if f.perm is None or f.perm.shape != (n,):
             f.perm = torch.zeros(n, dtype=torch.int64)
         f._g, f._g_buf = _Graph(), b
@@ -158,3 +159,14 @@ def test_rollout_steps_through_a_replaced_step(pkg, monkeypatch, where):
     t.t_dev, t.next_obs = torch.zeros(1, dtype=torch.int32), torch.zeros(6, 1800, dtype=torch.uint8)
     t._rollout_body()
     assert calls == ['step' if where else 'step_into'] * 4
+
+
+def test_update_refuses_rewards_of_another_size_than_the_graph(fast):
+    """The captured advantages hold T x N values."""
+    buf = ppo.RolloutBuffer(4, 512, device='cpu')
+    _ready(fast, buf, True)
+    fast.update(buf, generator=torch.Generator().manual_seed(1))
+    for name in ('rewards', 'values', 'dones'):
+        setattr(buf, name, torch.cat([getattr(buf, name)] * 2))
+    with pytest.raises(ValueError):
+        fast.update(buf, generator=torch.Generator().manual_seed(1))
