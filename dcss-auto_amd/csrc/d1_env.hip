@@ -523,9 +523,9 @@ __device__ __forceinline__ void generate_level(Ctx &x, uint64_t seed, uint32_t e
     }
 }
 
-// ---------------------------------------------------------------- prefetched load
-// A k_step workgroup runs several consecutive worlds; the next world's row is fetched into
-// registers while the current one steps, so its HBM latency is off the critical path.
+// ---------------------------------------------------------------- load
+// A world's row goes into registers by one set of loads when its wave starts it (step_worlds says
+// why not earlier) and is unpacked from there.
 // Lane l holds dword l of header + view (l < 24), its monster (l < max_m) and words
 // l + 64i of the viewed and floor rows; every lane holds the action and the active flag.
 // Addresses are clamped in bounds (the lanes past a field read a copy of its last element).

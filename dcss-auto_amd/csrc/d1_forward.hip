@@ -601,7 +601,7 @@ __global__ __launch_bounds__(256) void k_policy(const uint8_t *__restrict__ obs,
 // them. A wave then reads only its own row block's weight fragments, which go from L2 straight
 // to registers (a ring, three or five chunks ahead), while the observations, which every wave
 // needs, are widened once into fragment-ordered LDS. What bounds it is the chain of one
-// workgroup: all of W1 into its CU (928 KB, 6 us at the 64 B/clk of a CU's L1; counted, 1.16 MB of
+// workgroup: all of W1 into its CU (928 KB, 6 us at the 64 B/clk of a CU's L1; counted, 1.17 MB of
 // L1 misses a workgroup, no LDS bank conflict), the layers one after the other, the draw. MFMA is busy
 // 3.5 us of it. k_policy -> here, forward + sample, launches of one graph: 47.2 -> 14.0 us at 1,024
 // rows, 47.4 -> 16.0 at 8,192 (TB = 1), 48.5 -> 25.3 at 16,384 (TB = 2); with the autoregressive head

@@ -653,8 +653,9 @@ __device__ __forceinline__ void primitive_learn(LCtx &c, int d, const Aim &to, i
         if (movers) bfs(x, movers, imax(2, (maxspeed + 9) / 10));
         while (x.hp > 0 && ballot(x.lane < REQ && x.menergy >= 80)) {   // no reduction once nobody can act
             // the lane id opaque per act, so that the monster rules' lane-derived masks and
-            // addresses are recomputed in each act instead of held through the loop: 168 -> 121
-            // VGPRs, 3 -> 4 waves per SIMD, k_learn_step 0.903 -> 0.796 ms
+            // addresses are recomputed in each act instead of held through the loop (168 -> 121
+            // VGPRs, 3 -> 4 waves per SIMD, k_learn_step 0.903 -> 0.796 ms when it came in; the
+            // kernel is built for 5 waves, 96 VGPRs, since)
             {
                 int l = lane_id();
                 asm volatile("" : "+v"(l));
