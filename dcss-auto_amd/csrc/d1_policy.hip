@@ -286,7 +286,11 @@ int d1_gae(const float *reward, const uint8_t *done, const float *value, const f
         hipLaunchKernelGGL(kernel, dim3((n + 63) / 64), dim3(64 * waves), 0, (hipStream_t)stream, reward, done, value,
                            bootstrap, T, n, gamma, gamma_lambda, adv, returns);
     };
-    using namespace d1p;   // the smallest kernel whose waves hold T steps
+    using namespace d1p;
+    // The smallest kernel whose waves hold T steps. Lines measured at 64 and 65,536 envs: T = 1 on four
+    // steps a wave 1.7 and 1.9 us, on sixteen 2.1 and 2.4; T = 16 on one wave 2.7 and 4.1, on eight 3.5
+    // and 8.3; T = 32 on two 3.2 and 6.6, on eight 3.6 and 9.5; T = 64 on four 3.7 and 11.7, on eight
+    // 3.9 and 16.2.
     if (T <= 4) go(k_gae<1, 4>, 1);
     else if (T <= GC) go(k_gae<1, GC>, 1);
     else if (T <= 2 * GC) go(k_gae<2, GC>, 2);
